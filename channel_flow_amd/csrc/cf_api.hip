@@ -134,9 +134,11 @@ struct cf_ctx {
   hipStream_t aux[3] = {nullptr, nullptr, nullptr};
   hipEvent_t fork_ev = nullptr, join_ev[3] = {nullptr, nullptr, nullptr};
   long spin_limit = 1L << 22;
-  // what the sweep-order NL slots that the forward sweep hands across tiles
-  // hold between iterations: 1 the double sentinel, 2 the float one, 0 unknown
+  // what the pipelined sweeps' hand-off slots hold between iterations: 1 the
+  // double sentinel, 2 the float one, 0 unknown
   int hand_off = 0;
+  // the NL slots that the single-wave tiles hand across hold the sentinel
+  bool tiles_seeded = false;
   double* partial = nullptr;
   double* er_dev = nullptr;   // the norms, then the two sweep error flags
   double* er_host = nullptr;  // pinned copy of er_dev, read after each iteration
@@ -291,10 +293,10 @@ extern "C" int cf_create(const cf_params* p, cf_ctx** out) {
   g.dXI = p->deltaXI;
   g.dET = p->deltaET;
   g.dZT = p->deltaZT;
-  // 0 where the residual-corrected division is not guaranteed: plain division
-  g.rXI = cf::rcp_checked(p->deltaXI);
-  g.rET = cf::rcp_checked(p->deltaET);
-  g.rZT = cf::rcp_checked(p->deltaZT);
+  g.rXI = 1.0 / p->deltaXI;
+  g.rET = 1.0 / p->deltaET;
+  g.rZT = 1.0 / p->deltaZT;
+  g.fast_div = cf::rcp_checked(p->deltaXI) != 0.0 && cf::rcp_checked(p->deltaET) != 0.0 && cf::rcp_checked(p->deltaZT) != 0.0;
   c->hprof.assign((size_t)NPROF * g.Ym, 0.0);
   auto bail = [&](int code) {
     cf_destroy(c);
@@ -317,7 +319,7 @@ extern "C" int cf_create(const cf_params* p, cf_ctx** out) {
     // the reference leaves work arrays uninitialised; here they start at zero
     if (hipMemsetAsync(*f.ptr, 0, nf * f.n * sizeof(double), c->stream) != hipSuccess) return bail(CF_ERR_HIP);
   }
-  if (hipMalloc(&c->Sm, (size_t)cf::sweep_field_elems(g) * (cf::G_N + 15) * sizeof(double)) != hipSuccess)
+  if (hipMalloc(&c->Sm, (size_t)cf::sweep_buffer_elems(g) * sizeof(double)) != hipSuccess)
     return bail(CF_ERR_HIP);
   {
     int nTI, nTJ;
@@ -782,18 +784,26 @@ static int effective_schedule(const cf_ctx* c) { return (c->schedule != 1 && dia
 // (lagged neighbour planes, :521-559); this library holds one domain.
 static int sweep_pairs(const cf_ctx* c) { return c->sweep_reuse ? std::min(c->p.n_sweeps, 1) : c->p.n_sweeps; }
 
-// The forward tiled sweep needs its cross-tile NL slots at the sentinel, and
-// every backward tiled sweep leaves them so: they are seeded here only when
-// that is not known (a new context, a sweep that gave up), eagerly and never
-// inside a graph capture (cf_inner_iteration seeds before it captures)
+// The tiled sweeps need their cross-tile slots at the sentinel and leave them
+// so: they are seeded here only when that is not known (a new context, a sweep
+// that gave up; for the single-wave tiles, whose slots are NL itself, also
+// pipelined sweeps since), eagerly and never inside a graph capture
+// (cf_inner_iteration seeds before it captures)
 static void seed_hand_off(cf_ctx* c) {
   if (c->solver != 0 || effective_schedule(c) != 0) return;
   const int want = c->fp32 ? 2 : 1;
-  if (c->hand_off == want) return;
+  const bool tiles = c->schedule == 2;
+  if (tiles ? c->tiles_seeded : (c->hand_off == want && !c->tiles_seeded)) return;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(c->stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return;
-  cf::launch_seed_hand_off(c->stream, c->Sm, c->g, c->fp32);
+  if (tiles) {
+    cf::launch_seed_tiles(c->stream, c->Sm, c->g);
+    c->tiles_seeded = true;
+    return;
+  }
+  if (c->hand_off != want) cf::launch_seed_hand_off(c->stream, c->Sm, c->g, c->fp32);
   c->hand_off = want;
+  c->tiles_seeded = false;
 }
 
 static void sweeps(cf_ctx* c, double deltaT, const hipEvent_t* marks = nullptr, bool fuse_rhs = false) {
@@ -837,11 +847,13 @@ static int finish_iteration(cf_ctx* c, double er[5]) {
   int r = sync(c);
   if (r) {
     c->hand_off = 0;
+    c->tiles_seeded = false;
     return r;
   }
   for (int v = 0; v < 5; v++) er[v] = c->er_host[v];
   if (c->solver == 0 && effective_schedule(c) == 0 && (c->er_host[5] != 0. || c->er_host[6] != 0.)) {
     c->hand_off = 0;  // a sweep that gave up may leave slots without the sentinel
+    c->tiles_seeded = false;
     return fail(c, CF_ERR_TIMEOUT, "LU-SGS sweep: a tile waited past its bound for an upstream tile");
   }
   for (int v = 0; v < 5; v++)

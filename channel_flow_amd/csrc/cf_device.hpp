@@ -27,7 +27,8 @@ struct Geo {
   long plane;   // Ym * Zp
   long nf;      // Xnp * plane
   double dXI, dET, dZT;
-  double rXI, rET, rZT;  // rcp_checked of the spacings, for div_prof
+  double rXI, rET, rZT;  // RN(1/d) of the spacings
+  bool fast_div;         // all three meet div_const's bound (rcp_checked)
 };
 
 __device__ __forceinline__ long at(const Geo& g, int i, int j, int k) {
@@ -93,9 +94,18 @@ __host__ __device__ __forceinline__ double rcp_checked(double d) {
   return fabs(e) <= 0x1p-54 ? r : 0.0;
 }
 
-// x/d with a reciprocal from rcp_checked (0: plain division)
-__device__ __forceinline__ double div_prof(double x, double d, double r) {
-  return r != 0.0 ? div_const(x, d, r) : x / d;
+// x/d for any normal divisor d, with r = RN(1/d) as the division gives it:
+// one correction more than div_const.  q1 is x/d with an error of a few 2^-105
+// before its own rounding, so it is within one ulp whatever r's own error, its
+// remainder is exact and Markstein's theorem makes the result the correctly
+// rounded x/d, sign of a zero quotient included: the same bits as x / d while
+// the quotient and x times 2^-53 stay in the normal range.  Five operations
+// where the division takes about twelve: it pays where d has several
+// dividends.
+__device__ __forceinline__ double div_rn(double x, double d, double r) {
+  const double q0 = x * r;
+  const double q1 = fma(-fma(q0, d, -x), r, q0);
+  return fma(-fma(q1, d, -x), r, q1);
 }
 
 // 1/(K-1); |RKG (K-1) - 1| = 2^-54.3 meets the bound (checked on the host
@@ -395,12 +405,14 @@ enum DiagField : int {
   G_N
 };
 
-// x / rho and x / K: correctly rounded in FP64; in the FP32 sweeps, products
-// with the hardware reciprocal (1 ulp) and with 1/K, which the inexact inner
-// solve tolerates
-__device__ __forceinline__ double over_rho(double x, double rho) { return x / rho; }
-__device__ __forceinline__ float over_rho(float x, float rho) { return x * __builtin_amdgcn_rcpf(rho); }
-__device__ __forceinline__ double over_k(double x) { return x / KG; }
+// x / rho and x / K: correctly rounded in FP64, through the reciprocals; in
+// the FP32 sweeps, products with the hardware reciprocal (1 ulp) and with 1/K,
+// which the inexact inner solve tolerates.  rr = rcp_rho(rho), shared by the
+// quotients of one cell.
+constexpr double RK = 1.0 / KG;  // |RK KG - 1| = 2^-54.4 meets div_const's bound
+__device__ __forceinline__ double over_rho(double x, double rho, double rr) { return div_rn(x, rho, rr); }
+__device__ __forceinline__ float over_rho(float x, float, float rr) { return x * rr; }
+__device__ __forceinline__ double over_k(double x) { return div_const(x, KG, RK); }
 __device__ __forceinline__ float over_k(float x) { return x * float(1.0 / KG); }
 
 // x / y in the sweep's type: correctly rounded in FP64, reciprocal product in
@@ -408,17 +420,28 @@ __device__ __forceinline__ float over_k(float x) { return x * float(1.0 / KG); }
 __device__ __forceinline__ double sweep_div(double x, double y) { return x / y; }
 __device__ __forceinline__ float sweep_div(float x, float y) { return x * __builtin_amdgcn_rcpf(y); }
 
+// x/d by a spacing: FD when all three spacings meet div_const's bound (three
+// operations instead of five)
+template <bool FD>
+__device__ __forceinline__ double div_sp(double x, double d, double r) {
+  return FD ? div_const(x, d, r) : div_rn(x, d, r);
+}
+
+// the reciprocal that over_rho takes for the divisor rho
+__device__ __forceinline__ double rcp_rho(double rho) { return 1.0 / rho; }
+__device__ __forceinline__ float rcp_rho(float rho) { return __builtin_amdgcn_rcpf(rho); }
+
 // D^-1 = {d11, d22 (= d33 = d44), d51} of one cell from its spectral radii
-// (Dual_time_stepping.cpp:464-489), dinv_lam's expressions in its order;
-// rdXI.. are 1/dXI.. for the FP32 sweeps (unused in FP64)
-template <class R>
-__device__ __forceinline__ void diag_dinv(R beta, R rho, R lx, R ly, R lz, double dXI, double dET, double dZT,
-                                          double deltaT, R* d11, R* d22, R* d51) {
+// (Dual_time_stepping.cpp:464-489), dinv_lam's expressions in its order; the
+// FP32 sweeps multiply by the spacings' reciprocals
+template <bool FD, class R>
+__device__ __forceinline__ void diag_dinv(R beta, R rho, R lx, R ly, R lz, const Geo& g, double deltaT, R* d11,
+                                          R* d22, R* d51) {
   R lambda;
   if constexpr (sizeof(R) == sizeof(double))
-    lambda = lx / dXI + ly / dET + lz / dZT;
+    lambda = div_sp<FD>(lx, g.dXI, g.rXI) + div_sp<FD>(ly, g.dET, g.rET) + div_sp<FD>(lz, g.dZT, g.rZT);
   else
-    lambda = lx * R(1.0 / dXI) + ly * R(1.0 / dET) + lz * R(1.0 / dZT);
+    lambda = lx * R(1.0 / g.dXI) + ly * R(1.0 / g.dET) + lz * R(1.0 / g.dZT);
   const R dt = R(deltaT);
   *d11 = sweep_div(R(2) * dt, R(3) * beta + R(2) * lambda * dt);
   *d22 = sweep_div(R(2) * dt, R(3) + R(2) * lambda * dt);
@@ -430,9 +453,9 @@ __device__ __forceinline__ void diag_dinv(R beta, R rho, R lx, R ly, R lz, doubl
 // PD = 0.5*n_dd/rho (A+21, B+31, C+41) and P51 = 0.5*U*(K-1)*(beta-1)/rho/K
 // of one direction (Dual_time_stepping.cpp:751-811), in the reference's order
 template <class R>
-__device__ __forceinline__ void split_pd_p51(R n, R U, R beta, R rho, R* pd, R* p51) {
-  *pd = over_rho(R(0.5) * n, rho);
-  *p51 = over_k(over_rho(R(0.5) * U * R(KG - 1) * (beta - R(1)), rho));
+__device__ __forceinline__ void split_pd_p51(R n, R U, R beta, R rho, R rr, R* pd, R* p51) {
+  *pd = over_rho(R(0.5) * n, rho, rr);
+  *p51 = over_k(over_rho(R(0.5) * U * R(KG - 1) * (beta - R(1)), rho, rr));
 }
 
 struct DNb {  // one neighbour as seen along one direction

@@ -9,6 +9,7 @@
 #include "cf_kernels.hpp"
 
 #include <type_traits>
+#include <utility>
 
 namespace cf {
 
@@ -1147,6 +1148,15 @@ __device__ __forceinline__ long sk_at(const Sk& q, int tile, int s, int lane) {
   return ((long)tile * q.nsteps + s) * 64 + lane;
 }
 
+// Slots of 5 x 8 values per tile, edge and step, each in cache lines of its
+// own: the hand-off of the pipelined sweeps (edge 0 x, 1 y) and the compact
+// copy of the summary along x (edge 0: a = 7, edge 1: a = 0; P, beta, rho, U_x
+// and lambda_x by b), whose lanes are 64 bytes apart in the rows
+constexpr int HO_SLOT = 64;  // elements per slot (40 used)
+__host__ __device__ __forceinline__ long ho_at(const Sk& q, int tile, int edge, int s) {
+  return (((long)tile * 2 + edge) * q.nsteps + s) * HO_SLOT;
+}
+
 // thread (s, lane) of a block of 16 steps x 64 lanes -> cell; false if the
 // slot holds no interior cell
 __device__ __forceinline__ bool sk_cell(const Sk& q, const Geo& g, int tile, int s, int lane, int* i, int* j,
@@ -1181,6 +1191,22 @@ __device__ __forceinline__ void prep_summary(const double u5[5], const double* _
   }
 }
 
+// the summary row, and the x edges' compact copy
+template <class T>
+__device__ __forceinline__ void store_summary(T* __restrict__ S, T* __restrict__ E, const Sk& q, int tile, int s,
+                                              int lane, const double v[G_N]) {
+  const long o = sk_at(q, tile, s, lane);
+#pragma unroll
+  for (int r = 0; r < G_N; r++) S[r * q.nsk + o] = T(v[r]);
+  const int a = lane & 7;
+  if (a == 0 || a == TI - 1) {
+    T* e = E + ho_at(q, tile, a == 0, s) + (lane >> 3);
+    constexpr int f[5] = {G_P, G_BETA, G_RHO, G_UX, G_LX};
+#pragma unroll
+    for (int r = 0; r < 5; r++) e[8 * r] = T(v[f[r]]);
+  }
+}
+
 // A prep block covers PC steps of one tile.  Column (a, b) of the tile meets
 // cells k-2 = s - a - b at steps s0 .. s0+PC-1: one run of PC consecutive k,
 // which the block stages in LDS with coalesced loads; slot (s, lane) then
@@ -1209,7 +1235,7 @@ __device__ __forceinline__ void prep_stage(double (*L)[64][PCP], const double* _
 template <class T>
 __global__ void __launch_bounds__(256) k_sweep_prep(const double* __restrict__ Ui, const double* __restrict__ MR,
                                                     const double* __restrict__ prof, T* __restrict__ S,
-                                                    T* __restrict__ MRs, Geo g, Sk q) {
+                                                    T* __restrict__ MRs, T* __restrict__ E, Geo g, Sk q) {
   __shared__ double L[5][64][PCP];
   int bx, by, bz;
   xcd_block3(&bx, &by, &bz);
@@ -1225,8 +1251,7 @@ __global__ void __launch_bounds__(256) k_sweep_prep(const double* __restrict__ U
 #pragma unroll
     for (int f = 0; f < 5; f++) u5[f] = L[f][lane][t];
     prep_summary(u5, prof, g, j, v);
-#pragma unroll
-    for (int r = 0; r < G_N; r++) S[r * q.nsk + o] = T(v[r]);
+    store_summary(S, E, q, tile, s, lane, v);
   }
   __syncthreads();
   prep_stage(L, MR, g, q, tile, s0);
@@ -1258,7 +1283,8 @@ static_assert(64 * PR % PR_THREADS == 0, "whole cells per thread");
 template <class T>
 __global__ void __launch_bounds__(PR_THREADS) k_sweep_prep_rhs(const double* __restrict__ Ui, RhsIn rin,
                                                                const double* __restrict__ prof, T* __restrict__ S,
-                                                               T* __restrict__ MRs, Geo g, Sk q, double deltaT) {
+                                                               T* __restrict__ MRs, T* __restrict__ E, Geo g, Sk q,
+                                                               double deltaT) {
   __shared__ double L[5][64][PRP];
   int bx, by, bz;
   xcd_block3(&bx, &by, &bz);
@@ -1309,8 +1335,7 @@ __global__ void __launch_bounds__(PR_THREADS) k_sweep_prep_rhs(const double* __r
 #pragma unroll
     for (int f = 0; f < 5; f++) u5[f] = L[f][lane][t];
     prep_summary(u5, prof, g, j, v);
-#pragma unroll
-    for (int r = 0; r < G_N; r++) S[r * q.nsk + o] = T(v[r]);
+    store_summary(S, E, q, tile, s, lane, v);
   }
 }
 
@@ -1327,16 +1352,16 @@ __global__ void __launch_bounds__(1024) k_sk_to_natural(const T* __restrict__ sr
   for (int v = 0; v < nfields; v++) dst[v * g.nf + c] = double(src[v * q.nsk + o]);
 }
 
-// The NL slots a forward sweep hands across tiles (lanes on a tile's high x
-// or y edge, every step) set to the sentinel.  Each backward sweep sets every
-// such slot it has read back to the sentinel, so this runs only when the
-// slots may hold anything else: a new buffer, or after a sweep that gave up.
-template <class T>
-__global__ void __launch_bounds__(256) k_seed_hand_off(T* __restrict__ NLs, Sk q) {
+// The NL slots that k_sweep_tiles' forward sweep hands across tiles (lanes on
+// a tile's high x or y edge, every step) set to the sentinel.  Its backward
+// sweep sets every such slot it has read back to the sentinel, so this runs
+// only when the slots may hold anything else: a new buffer, after a sweep
+// that gave up, or after pipelined sweeps, which fill NL.
+__global__ void __launch_bounds__(256) k_seed_tiles(double* __restrict__ NLs, Sk q) {
   const int lane = threadIdx.x & 63, s = blockIdx.x * 4 + (threadIdx.x >> 6), tile = blockIdx.y;
   if (s >= q.nsteps || ((lane & 7) != TI - 1 && (lane >> 3) != TJ - 1)) return;
   const long o = sk_at(q, tile, s, lane);
-  const T sv = sentinel_value<T>();
+  const double sv = sentinel_value<double>();
 #pragma unroll
   for (int v = 0; v < 5; v++) NLs[v * q.nsk + o] = sv;
 }
@@ -1382,7 +1407,7 @@ __device__ __forceinline__ DNb dnb_at(const double* __restrict__ S, long nsk, lo
   c.beta = S[G_BETA * nsk + p];
   c.U = S[(G_UX + 2 * d) * nsk + p];
   c.lam = S[(G_LX + 2 * d) * nsk + p];
-  split_pd_p51(n, c.U, c.beta, rho, &c.pd, &c.p51);
+  split_pd_p51(n, c.U, c.beta, rho, rcp_rho(rho), &c.pd, &c.p51);
   return c;
 }
 
@@ -1544,11 +1569,10 @@ __global__ void __launch_bounds__(64) k_sweep_tiles(const double* __restrict__ S
       double L[5];
 #pragma unroll
       for (int v = 0; v < 5; v++)
-        L[v] = div_prof(acc[0][v], g.dXI, g.rXI) + div_prof(acc[1][v], g.dET, g.rET) +
-               div_prof(acc[2][v], g.dZT, g.rZT);
+        L[v] = div_rn(acc[0][v], g.dXI, g.rXI) + div_rn(acc[1][v], g.dET, g.rET) + div_rn(acc[2][v], g.dZT, g.rZT);
       double d11, d22, d51;
-      diag_dinv(cur.own[G_BETA], cur.own[G_RHO], cur.own[G_LX], cur.own[G_LY], cur.own[G_LZ], g.dXI, g.dET, g.dZT,
-                deltaT, &d11, &d22, &d51);
+      diag_dinv<false>(cur.own[G_BETA], cur.own[G_RHO], cur.own[G_LX], cur.own[G_LY], cur.own[G_LZ], g, deltaT, &d11,
+                       &d22, &d51);
       const double* M = cur.src;
       double out[5];
       if (FWD) {
@@ -1589,7 +1613,7 @@ __global__ void __launch_bounds__(64) k_sweep_tiles(const double* __restrict__ S
 #pragma unroll
       for (int d = 0; d < 2; d++) {
         double pd, p51;
-        split_pd_p51(dn[d], cur.own[G_UX + 2 * d], cur.own[G_BETA], cur.own[G_RHO], &pd, &p51);
+        split_pd_p51(dn[d], cur.own[G_UX + 2 * d], cur.own[G_BETA], cur.own[G_RHO], rcp_rho(cur.own[G_RHO]), &pd, &p51);
         lds[cb][8 + 4 * d][lane] = cur.own[G_UX + 2 * d];
         lds[cb][9 + 4 * d][lane] = cur.own[G_LX + 2 * d];
         lds[cb][10 + 4 * d][lane] = pd;
@@ -1600,7 +1624,7 @@ __global__ void __launch_bounds__(64) k_sweep_tiles(const double* __restrict__ S
       zc.beta = cur.own[G_BETA];
       zc.U = cur.own[G_UZ];
       zc.lam = cur.own[G_LZ];
-      split_pd_p51(dn[2], zc.U, zc.beta, cur.own[G_RHO], &zc.pd, &zc.p51);
+      split_pd_p51(dn[2], zc.U, zc.beta, cur.own[G_RHO], rcp_rho(cur.own[G_RHO]), &zc.pd, &zc.p51);
     }
     // one wave per block: LDS writes of this step are complete and ordered
     // before the next step's reads
@@ -1612,26 +1636,48 @@ __global__ void __launch_bounds__(64) k_sweep_tiles(const double* __restrict__ S
 
 // ---------------------------------------------------------------------------
 // Pipelined tiled sweep: the same tiles, steps and arithmetic as
-// k_sweep_tiles, with the loads and the neighbour coefficients taken off the
-// compute wave.  A block is four waves meeting at one LDS-only barrier per
-// step (loads stay in flight across steps):
-//   wave 0  computes one cell per lane and step from LDS only;
-//   wave 1  loads the lane cells' summaries QS steps ahead and turns them
-//           into the x and y split-Jacobian entries their downstream
-//           neighbours use (SplitCoef, diag_coef);
-//   wave 2  loads MR (forward) or NL (backward) and the summaries, and forms
-//           D^-1 and the z entries;
-//   wave 3  fetches the cross-tile halo: the neighbour tile's summary (as
-//           SplitCoef) and its NL/NR, polled until the sentinel is overwritten,
-//           QD steps ahead.
-// LDS holds three step slots of per-lane data; slot s-1 carries the
-// neighbour entries of step s, with the halo in columns 64..71 (x: by b,
-// y: by a) so that every lane reads its neighbours at fixed offsets.
+// k_sweep_tiles, spread over the ten waves of a block that meet at one
+// LDS-only barrier per step (loads stay in flight across steps).  The sweep
+// is a chain of dependent steps, so its time is the number of steps on the
+// longest path times the work of the busiest wave (and SIMD) per step; every
+// wave does one short job:
+//   waves 0-3   load the rows of every fourth step and form, over four steps'
+//               time, D^-1 and the split-Jacobian entries (SplitCoef,
+//               diag_coef) that the cells' downstream neighbours use;
+//   waves 4, 5  compute one cell per lane and step from LDS only, wave 4 the
+//               components P and T (0, 4), wave 5 the velocities (1, 2, 3):
+//               each component reads at most two others of a neighbour, and
+//               those cross between the two waves with the neighbours' values;
+//   waves 6, 7  poll the cross-tile neighbours' outputs of the even (odd) steps;
+//   wave 8      writes the outputs to their rows;
+//   wave 9      the split-Jacobian entries of the cross-tile neighbours, four
+//               steps at a time (16 cells a step).
+// Waves w, w + 4 and w + 8 share a SIMD.  What bounds it: at 64^3 the step, at
+// 256x192x256 (FP64) also the 2.2 GB a sweep moves.  Measured, forward /
+// backward, against four waves per block (one computing all five components,
+// two loading, one polling two steps ahead; hand-off through the NL and NR
+// rows): 64^3 FP64 156 / 151 -> 105 / 107 us, FP32 128 / 124 -> 83 / 84 us;
+// 97x75x130 341 / 328 -> 184 / 179 and 205 / 195 -> 142 / 135 us; 256x192x256
+// 915 / 838 -> 639 / 635 and 655 / 640 -> 485 / 475 us.  Steps that did not
+// pay: two loader waves of every second step (64^3 144 us: each then takes
+// longer than the compute waves), a wave per direction and one for D^-1 (131
+// us), polling 4 or 8 steps ahead (120, 141 us), one polling wave (104 us at
+// 64^3, but 795 us at 256x192x256), two tiles per CU (no change).
+// LDS holds four step slots of per-lane data; slot s-1 carries the neighbour
+// entries of step s, with the halo in columns 64..71 (x: by b, y: by a) so
+// that every lane reads its neighbours at fixed offsets.
+//
+// Hand-off between tiles: slot s of a tile's x (or y) edge holds the 5 x 8
+// outputs its downstream tile needs from step s, contiguous, in a buffer of
+// its own.  The compute waves write a slot with agent-scope relaxed stores as
+// soon as they have the values; the consumer's wave 6 or 7 re-reads it until no
+// value is the sentinel, then its wave 8 sets it back to the sentinel.  So
+// the buffer holds sentinels only between sweeps, whatever their direction,
+// and the output rows themselves are ordinary stores.  A slot has 64
+// elements, so no cache line holds values of two steps.
 // ---------------------------------------------------------------------------
-// Lookaheads measured at 256x192x256 with one tile per CU: QD = 1 and 3
-// were slower than 2, QS = 2 and 4 equal to 3.
-constexpr int PIPE_QS = 3;  // own-field lookahead (steps)
-constexpr int PIPE_QD = 2;  // halo lookahead (steps)
+constexpr int PIPE_THREADS = 640;
+constexpr int PIPE_SLOTS = 4;  // step slots in LDS
 constexpr int PO_D11 = 0, PO_D22 = 1, PO_D51 = 2, PO_M = 3, PO_Z = 8, PO_N = 14;  // rows of PipeLds::own
 
 __device__ __forceinline__ void lds_barrier() {
@@ -1640,31 +1686,49 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// f(0), f(1), .. f(N-1) in turn, again and again, until one returns false;
+// the argument is an integral_constant, so that every register and LDS slot
+// index is a constant.  for_each calls each once.
+template <class F, int... K>
+__device__ __forceinline__ void cycle_seq(F f, std::integer_sequence<int, K...>) {
+  while ((f(std::integral_constant<int, K>{}) && ...)) {
+  }
+}
+template <int N, class F>
+__device__ __forceinline__ void cycle(F f) {
+  cycle_seq(f, std::make_integer_sequence<int, N>{});
+}
+template <class F, int... K>
+__device__ __forceinline__ void each_seq(F f, std::integer_sequence<int, K...>) {
+  (f(std::integral_constant<int, K>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void for_each(F f) {
+  each_seq(f, std::make_integer_sequence<int, N>{});
+}
+template <int N>
+using Int = std::integral_constant<int, N>;
+
+// an ordinary load that the compiler leaves where it is written: without
+// this it sinks a load of a later step to the step that uses it
+template <class T>
+__device__ __forceinline__ T ld_here(const T* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
+
 // T: the sweep's arithmetic and storage type (double, or float for the FP32
 // inner solve)
 template <class T>
-struct PipeData {
-  T own[3][PO_N][64];  // D11 D22 D51, MR or NL (5), z SplitCoef (6) of the lane cells
-  T xc[3][6][72];      // x SplitCoef: lanes, then the x halo by b
-  T yc[3][6][72];      // y SplitCoef: lanes, then the y halo by a
-  T N[2][5][80];       // outputs of the previous step: lanes, x halo by b (64+), y halo by a (72+)
+struct PipeLds {
+  T own[PIPE_SLOTS][PO_N][64];  // D11 D22 D51, MR or NL (5), z SplitCoef (6) of the lane cells
+  T xc[PIPE_SLOTS][6][72];      // x SplitCoef: lanes, then the x halo by b
+  T yc[PIPE_SLOTS][6][72];      // y SplitCoef: lanes, then the y halo by a
+  T N[2][5][80];                // outputs of the previous step: lanes, x halo by b (64+), y halo by a (72+)
   int ticket;
 };
 
-// One tile per CU.  The block reserves more than half of the CU's 160 KB of
-// LDS so that no second sweep block shares the CU: co-resident tiles slow
-// each other's compute wave, which is on the critical path, by more than the
-// extra tiles in flight gain (256x192x256, one forward sweep: 3.46 ms with
-// three tiles per CU, 2.79 ms with two, 2.24 ms with one).
-constexpr int PIPE_LDS_BYTES = 82 * 1024;
-template <class T>
-struct PipeLds : PipeData<T> {
-  char reserve[PIPE_LDS_BYTES - sizeof(PipeData<T>)];
-};
-static_assert(sizeof(PipeLds<double>) > 80 * 1024 && sizeof(PipeLds<float>) > 80 * 1024, "one sweep block per CU");
-
-template <class T>
-__device__ __forceinline__ void coef_store(T (&row)[6][72], int col, const SplitCoefT<T>& c) {
+template <class T, int W>
+__device__ __forceinline__ void coef_store(T (*row)[W], int col, const SplitCoefT<T>& c) {
   row[0][col] = c.c11;
   row[1][col] = c.c1q;
   row[2][col] = c.c22;
@@ -1673,24 +1737,42 @@ __device__ __forceinline__ void coef_store(T (&row)[6][72], int col, const Split
   row[5][col] = c.p51;
 }
 
-template <class T>
-__device__ __forceinline__ SplitCoefT<T> coef_load(const T (&row)[6][72], int col) {
-  return SplitCoefT<T>{row[0][col], row[1][col], row[2][col], row[3][col], row[4][col], row[5][col]};
+// A neighbour's contribution to the components a compute wave owns: those of
+// diag_apply, expression by expression.  PT: components 0 and 4 (o[0], o[1]);
+// otherwise components 1, 2, 3.
+template <int D, bool FWD, bool PT, int W, class T>
+__device__ __forceinline__ void apply_part(T (*c)[W], int col, const T N[5], T o[3]) {
+  constexpr int q = D + 1;
+  const T c22 = c[2][col];
+  if constexpr (PT) {
+    const T c11 = c[0][col], c1q = c[1][col], c5q = c[3][col], p51 = c[5][col];
+    if (FWD) {
+      o[0] = -c11 * N[0] - c1q * N[q];
+      o[1] = -p51 * N[0] - c5q * N[q] - c22 * N[4];
+    } else {
+      o[0] = +c11 * N[0] + c1q * N[q];
+      o[1] = +p51 * N[0] + c5q * N[q] + c22 * N[4];
+    }
+  } else {
+    const T pd = c[4][col];
+#pragma unroll
+    for (int m = 1; m <= 3; m++) {
+      if (FWD)
+        o[m - 1] = m == q ? -pd * N[0] - c22 * N[m] : -(c22 * N[m]);
+      else
+        o[m - 1] = m == q ? +pd * N[0] + c22 * N[m] : c22 * N[m];
+    }
+  }
 }
 
-// x/d by a spacing: FD when all three spacings have checked reciprocals
-template <bool FD>
-__device__ __forceinline__ double div_sp(double x, double d, double r) {
-  if (FD) return div_const(x, d, r);
-  return x / d;
-}
-
-// wave 0: one cell per lane and step, inputs from LDS only.  In FP32 the
-// divisions by the spacings become products with their float reciprocals.
-template <bool FWD, bool FD, class T>
-__device__ void pipe_compute(PipeLds<T>& L, T* __restrict__ SRC, T* __restrict__ DST, T* __restrict__ AUX,
-                             const Geo& g, const Sk& q, int tile, int TX, int TY) {
+// waves 4 and 5: one cell per lane and step, inputs from LDS only.  In FP32
+// the divisions by the spacings become products with their float reciprocals.
+template <bool FWD, bool FD, bool PT, class T>
+__device__ __forceinline__ void pipe_compute(PipeLds<T>& L, T* __restrict__ H, const Geo& g, const Sk& q, int tile,
+                                             int TX, int TY) {
   constexpr bool F64 = std::is_same<T, double>::value;
+  constexpr int NC = PT ? 2 : 3;
+  constexpr int comp[3] = {PT ? 0 : 1, PT ? 4 : 2, 3};
   const int lane = threadIdx.x & 63;
   const int a = lane & 7, b = lane >> 3;
   const int i = 3 + TX * TI + a, j = 2 + TY * TJ + b;
@@ -1701,372 +1783,457 @@ __device__ void pipe_compute(PipeLds<T>& L, T* __restrict__ SRC, T* __restrict__
   const bool y_dom = FWD ? j - 1 >= 2 : j + 1 <= g.ny;
   const bool x_in = FWD ? a > 0 : a < TI - 1;
   const bool y_in = FWD ? b > 0 : b < TJ - 1;
+  // some cell of the tile has no x (y) neighbour: the same for all lanes
+  const bool rim = FWD ? TX == 0 || TY == 0 : TX + 1 == q.nTI || tile + q.nTI >= q.ntiles;
   // neighbour columns: in-tile lanes or the halo
   const int xi = x_in ? (FWD ? lane - 1 : lane + 1) : 64 + b;
   const int yi = y_in ? (FWD ? lane - 8 : lane + 8) : 64 + a;
   const int yiN = y_in ? yi : 72 + a;
-  const long nf = q.nsk;
-  const bool edge_fwd = a == TI - 1 || b == TJ - 1;
-  const bool edge_bwd = a == 0 || b == 0;
-  const T sv = sentinel_value<T>();
+  // lanes whose outputs the downstream tiles read
+  const bool hx = FWD ? a == TI - 1 && TX + 1 < q.nTI : a == 0 && TX > 0;
+  const bool hy = FWD ? b == TJ - 1 && tile + q.nTI < q.ntiles : b == 0 && TY > 0;
+  T* Hx = H + ho_at(q, tile, 0, 0) + b;
+  T* Hy = H + ho_at(q, tile, 1, 0) + a;
   const float fXI = float(1.0 / g.dXI), fET = float(1.0 / g.dET), fZT = float(1.0 / g.dZT);
   T zN[5] = {0, 0, 0, 0, 0};
-  int cs = 0, ps = 2;
+  int tau = 0;
   lds_barrier();  // step 0 inputs are in LDS
-  for (int tau = 0; tau < nsteps; tau++) {
+  cycle<PIPE_SLOTS>([&](auto k) -> bool {
+    constexpr int cs = decltype(k)::value, ps = (cs + PIPE_SLOTS - 1) % PIPE_SLOTS, nw = cs & 1, nr = nw ^ 1;
     const int kk = tau - off;
-    const int nr = (tau & 1) ^ 1, nw = tau & 1;
     if (col && kk >= 0 && kk < Nz) {
-      const T d11 = L.own[cs][PO_D11][lane], d22 = L.own[cs][PO_D22][lane], d51 = L.own[cs][PO_D51][lane];
-      T M[5];
+      const T d22 = L.own[cs][PO_D22][lane];
+      T d11 = 0, d51 = 0;
+      if constexpr (PT) {
+        d11 = L.own[cs][PO_D11][lane];
+        d51 = L.own[cs][PO_D51][lane];
+      }
+      T M[NC];
 #pragma unroll
-      for (int v = 0; v < 5; v++) M[v] = L.own[cs][PO_M + v][lane];
+      for (int v = 0; v < NC; v++) M[v] = L.own[cs][PO_M + comp[v]][lane];
       // both neighbours' inputs are read unconditionally (the indices are
       // inside the LDS rows for every lane), so the x and y reads share one
-      // LDS round trip; a neighbour outside the domain contributes zero
+      // LDS round trip; a neighbour outside the domain contributes zero.
+      // Components that apply_part does not use are not read.
       T Nx[5], Ny[5];
 #pragma unroll
       for (int v = 0; v < 5; v++) {
         Nx[v] = L.N[nr][v][xi];
         Ny[v] = L.N[nr][v][yiN];
       }
-      const SplitCoefT<T> cx = coef_load(L.xc[ps], xi), cy = coef_load(L.yc[ps], yi);
-      // the z neighbour is this lane's cell of the previous step: its split
-      // Jacobian is still in that step's own slot (the loaders fill another)
-      const SplitCoefT<T> cz = {L.own[ps][PO_Z + 0][lane], L.own[ps][PO_Z + 1][lane], L.own[ps][PO_Z + 2][lane],
-                                L.own[ps][PO_Z + 3][lane], L.own[ps][PO_Z + 4][lane], L.own[ps][PO_Z + 5][lane]};
-      T acc[3][5];
-      diag_apply<0, FWD>(cx, Nx, acc[0]);
-      diag_apply<1, FWD>(cy, Ny, acc[1]);
+      // the z neighbour is this lane's cell of the previous step: the
+      // component of the other compute wave comes through LDS, and its split
+      // Jacobian is still in that step's own slot (the loaders fill others)
+      if constexpr (PT)
+        zN[3] = L.N[nr][3][lane];
+      else
+        zN[0] = L.N[nr][0][lane];
+      T ax[3], ay[3], az[3];
+      apply_part<0, FWD, PT>(L.xc[ps], xi, Nx, ax);
+      apply_part<1, FWD, PT>(L.yc[ps], yi, Ny, ay);
+      apply_part<2, FWD, PT>(&L.own[ps][PO_Z], lane, zN, az);
+      if (rim) {
 #pragma unroll
-      for (int v = 0; v < 5; v++) {
-        acc[0][v] = x_dom ? acc[0][v] : T(0);
-        acc[1][v] = y_dom ? acc[1][v] : T(0);
+        for (int v = 0; v < NC; v++) {
+          ax[v] = x_dom ? ax[v] : T(0);
+          ay[v] = y_dom ? ay[v] : T(0);
+        }
       }
-      diag_apply<2, FWD>(cz, zN, acc[2]);
+      if (tau < TI + TJ - 1) {  // a lane's first cell is at step off < TI + TJ - 1
 #pragma unroll
-      for (int v = 0; v < 5; v++) acc[2][v] = kk > 0 ? acc[2][v] : T(0);
-      T Lv[5];
+        for (int v = 0; v < NC; v++) az[v] = kk > 0 ? az[v] : T(0);
+      }
+      T Lv[NC];
 #pragma unroll
-      for (int v = 0; v < 5; v++) {
+      for (int v = 0; v < NC; v++) {
         if constexpr (F64)
-          Lv[v] = div_sp<FD>(acc[0][v], g.dXI, g.rXI) + div_sp<FD>(acc[1][v], g.dET, g.rET) +
-                  div_sp<FD>(acc[2][v], g.dZT, g.rZT);
+          Lv[v] = div_sp<FD>(ax[v], g.dXI, g.rXI) + div_sp<FD>(ay[v], g.dET, g.rET) + div_sp<FD>(az[v], g.dZT, g.rZT);
         else
-          Lv[v] = acc[0][v] * fXI + acc[1][v] * fET + acc[2][v] * fZT;
+          Lv[v] = ax[v] * fXI + ay[v] * fET + az[v] * fZT;
       }
-      T out[5];
-      if (FWD) {
-        out[0] = d11 * (M[0] - Lv[0]);
-        out[1] = d22 * (M[1] - Lv[1]);
-        out[2] = d22 * (M[2] - Lv[2]);
-        out[3] = d22 * (M[3] - Lv[3]);
-        out[4] = d51 * (M[0] - Lv[0]) + d22 * (M[4] - Lv[4]);
+      T out[NC];
+      if constexpr (PT) {
+        if (FWD) {
+          out[0] = d11 * (M[0] - Lv[0]);
+          out[1] = d51 * (M[0] - Lv[0]) + d22 * (M[1] - Lv[1]);
+        } else {
+          out[0] = M[0] - d11 * Lv[0];
+          out[1] = M[1] - (d51 * Lv[0] + d22 * Lv[1]);
+        }
       } else {
-        out[0] = M[0] - d11 * Lv[0];
-        out[1] = M[1] - d22 * Lv[1];
-        out[2] = M[2] - d22 * Lv[2];
-        out[3] = M[3] - d22 * Lv[3];
-        out[4] = M[4] - (d51 * Lv[0] + d22 * Lv[4]);
+#pragma unroll
+        for (int v = 0; v < NC; v++) out[v] = FWD ? d22 * (M[v] - Lv[v]) : M[v] - d22 * Lv[v];
       }
-      const long c = sk_at(q, tile, FWD ? tau : nsteps - 1 - tau, lane);
+      // downstream tiles first: they are waiting
+      if (hx) {
 #pragma unroll
-      for (int v = 0; v < 5; v++) st_coherent(DST + v * nf + c, out[v]);
-      if (FWD && edge_bwd) {
-        // the backward sweep that follows hands these NR slots across tiles
-#pragma unroll
-        for (int v = 0; v < 5; v++) AUX[v * nf + c] = sv;
+        for (int v = 0; v < NC; v++) st_coherent(Hx + comp[v] * 8, out[v]);
       }
-      if (!FWD && edge_fwd) {
-        // this NL slot has been consumed; the next forward sweep hands it on
+      if (hy) {
 #pragma unroll
-        for (int v = 0; v < 5; v++) SRC[v * nf + c] = sv;
+        for (int v = 0; v < NC; v++) st_coherent(Hy + comp[v] * 8, out[v]);
       }
 #pragma unroll
-      for (int v = 0; v < 5; v++) {
-        L.N[nw][v][lane] = out[v];
-        zN[v] = out[v];
+      for (int v = 0; v < NC; v++) {
+        L.N[nw][comp[v]][lane] = out[v];
+        zN[comp[v]] = out[v];
       }
     }
-    ps = cs;
-    cs = cs == 2 ? 0 : cs + 1;
+    Hx += HO_SLOT;
+    Hy += HO_SLOT;
     lds_barrier();
-  }
+    return ++tau < nsteps;
+  });
 }
 
-// Loader step loop shared by the loader waves: before barrier tau+1 the data
-// of step tau+1 goes from register slot (tau+1) % Q to LDS and the slot is
-// refilled with step tau+1+Q.  Every iteration of the main loop issues the
-// same loads (the step index is clamped, so addresses stay inside the
-// arrays), which lets the compiler count the loads in flight exactly and wait
-// only for the oldest slot; the guarded remainder runs after it.
-template <int Q, class Consume, class Issue>
-__device__ __forceinline__ void pipe_loader_loop(int nsteps, Consume consume, Issue issue) {
-  static_assert(Q >= 1 && Q <= 8, "lookahead");
-  int t0 = 0;
-  for (; t0 + Q <= nsteps; t0 += Q) {
-#pragma unroll
-    for (int k = 0; k < Q; k++) {
-      consume(t0 + k + 1, (k + 1) % Q);
-      issue(t0 + k + 1 + Q, (k + 1) % Q);
-      lds_barrier();
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < Q; k++) {
-    if (t0 + k < nsteps) {
-      consume(t0 + k + 1, (k + 1) % Q);
-      lds_barrier();
-    }
-  }
+// the split-Jacobian entries of one cell along x (along_x) or y, z from its
+// summary; rr = rcp_rho(rho), T = P / rho
+template <bool FWD, class T>
+__device__ __forceinline__ SplitCoefT<T> coef_of(T P, T beta, T rho, T rr, T Tc, T U, T lam, T n, bool along_x) {
+  T pd, p51;
+  split_pd_p51(n, U, beta, rho, rr, &pd, &p51);
+  SplitCoefT<T> c = diag_coef<1, FWD>(P, Tc, beta, U, lam, pd, p51, n);
+  if (along_x) c.c5q = diag_coef<0, FWD>(P, Tc, beta, U, lam, pd, p51, n).c5q;
+  return c;
 }
 
-template <int Q, int NF, class T>
-struct Slots {
-  T v[Q][NF];
-  __device__ __forceinline__ void put(int sl, const T (&d)[NF]) {
+// waves 0 .. 3 (r): the steps s = r (mod 4), each over four steps' time: D^-1
+// at step s - 4 and to LDS with MR (forward) or NL (backward) at step s - 3,
+// the x and y split-Jacobian entries at step s - 2, the z ones at step s - 1;
+// then the loads of step s + 8.  A slot's D^-1 and M rows are last read at
+// step s - 4, its entries at step s - 3.  Every turn issues the same loads
+// (the step is clamped), so the compiler counts the loads in flight exactly
+// and waits only for the oldest.
+template <bool FWD, bool FD, class T>
+__device__ __forceinline__ void pipe_loader(PipeLds<T>& L, const T* __restrict__ S, const T* __restrict__ SRC,
+                                            const double* __restrict__ prof, const Geo& g, const Sk& q, int tile,
+                                            int TY, int r, double deltaT) {
+  static_assert(PIPE_SLOTS == 4, "one loader wave per slot");
+  constexpr int NF = 5 + G_N, F = 5;  // SRC0..4, then the summary
+  const int lane = threadIdx.x & 63;
+  const int nsteps = q.nsteps;
+  const long nf = q.nsk, row0 = (long)tile * nsteps * 64;
+  // metric of the lane's j (clamped for columns outside the domain)
+  const int j = min(2 + TY * TJ + (lane >> 3), g.ny);
+  const T nx = T(pf(prof, g.Ym, SET_C, 1, j)), ny = T(pf(prof, g.Ym, SET_C, 5, j)),
+          nz = T(pf(prof, g.Ym, SET_C, 9, j));
+  T(*own)[64] = L.own[r];
+  T buf[2][NF];
+  T d11 = 0, d22 = 0, d51 = 0, rr = 0, Tc = 0;
+  auto issue = [&](int s, auto sl) {
+    const int sc = min(s, nsteps - 1);
+    const long c = row0 + (long)(FWD ? sc : nsteps - 1 - sc) * 64;
 #pragma unroll
-    for (int k = 0; k < Q; k++)
-      if (k == sl) {
+    for (int f = 0; f < NF; f++) buf[sl][f] = ld_here((f < F ? SRC + c + (long)f * nf : S + c + (long)(f - F) * nf) + lane);
+  };
+  auto part = [&](auto which, auto sl) {
+    constexpr int W = decltype(which)::value;
+    const T(&d)[NF] = buf[sl];
+    const T P = d[F + G_P], be = d[F + G_BETA], rho = d[F + G_RHO];
+    if constexpr (W == 0) {
+      diag_dinv<FD>(be, rho, d[F + G_LX], d[F + G_LY], d[F + G_LZ], g, deltaT, &d11, &d22, &d51);
+    } else if constexpr (W == 1) {
+      own[PO_D11][lane] = d11;
+      own[PO_D22][lane] = d22;
+      own[PO_D51][lane] = d51;
 #pragma unroll
-        for (int f = 0; f < NF; f++) v[k][f] = d[f];
-      }
+      for (int f = 0; f < F; f++) own[PO_M + f][lane] = d[f];
+      rr = rcp_rho(rho);
+      Tc = over_rho(P, rho, rr);
+    } else if constexpr (W == 2) {
+      coef_store(L.xc[r], lane, coef_of<FWD>(P, be, rho, rr, Tc, d[F + G_UX], d[F + G_LX], nx, true));
+      coef_store(L.yc[r], lane, coef_of<FWD>(P, be, rho, rr, Tc, d[F + G_UY], d[F + G_LY], ny, false));
+    } else {
+      coef_store(&own[PO_Z], lane, coef_of<FWD>(P, be, rho, rr, Tc, d[F + G_UZ], d[F + G_LZ], nz, false));
+    }
+  };
+  issue(r, Int<0>{});
+  issue(r + 4, Int<1>{});
+  for_each<4>([&](auto k) { part(k, Int<0>{}); });
+  issue(r + 8, Int<0>{});
+  lds_barrier();
+  int tau = 0;
+  for (; tau < r; tau++) lds_barrier();  // nsteps > 3 in every grid
+  cycle<8>([&](auto k) -> bool {
+    constexpr int W = decltype(k)::value % 4;
+    const Int<1 - decltype(k)::value / 4> sl;
+    part(Int<W>{}, sl);
+    if constexpr (W == 3) issue(tau + 9, sl);  // the step at hand is tau + 1
+    lds_barrier();
+    return ++tau < nsteps;
+  });
+}
+
+// The halo has 16 consumer lanes of the compute waves: 0..7 on the x edge
+// (b = c) and 8..15 on the y edge (a = c - 8).
+template <bool FWD>
+struct HaloLane {
+  int dir, idx, a, b, off;
+  bool ok;  // the consumer is a cell of the domain and has this neighbour
+  __device__ __forceinline__ HaloLane(int dir_, int idx_, const Geo& g, int TX, int TY) : dir(dir_), idx(idx_) {
+    a = dir == 0 ? (FWD ? 0 : TI - 1) : idx;
+    b = dir == 0 ? idx : (FWD ? 0 : TJ - 1);
+    const int i = 3 + TX * TI + a, j = 2 + TY * TJ + b;
+    const bool dom = dir == 0 ? (FWD ? i - 1 >= 3 : i + 1 <= g.gend) : (FWD ? j - 1 >= 2 : j + 1 <= g.ny);
+    ok = i <= g.gend && j <= g.ny && dom;
+    off = FWD ? a + b : (TI - 1 - a) + (TJ - 1 - b);
   }
-  __device__ __forceinline__ void get(int sl, T (&d)[NF]) const {
-#pragma unroll
-    for (int f = 0; f < NF; f++) d[f] = v[0][f];
-#pragma unroll
-    for (int k = 1; k < Q; k++)
-      if (k == sl) {
-#pragma unroll
-        for (int f = 0; f < NF; f++) d[f] = v[k][f];
-      }
+  __device__ __forceinline__ bool live(int sig, const Sk& q) const {
+    const int kk = sig - off;
+    return ok && kk >= 0 && kk < q.Nz;
   }
 };
 
-// waves 1 and 2: the lane cells' fields QS steps ahead.  XY (wave 1): P,
-// beta, rho and the x, y summaries -> x, y SplitCoef.  Otherwise (wave 2): SRC
-// and P, beta, rho, the z summary and lambda -> D^-1, SRC and the z SplitCoef
-// in the own rows.
-template <bool FWD, bool XY, int QS, class T>
-__device__ void pipe_own_loader(PipeLds<T>& L, const T* __restrict__ S, const T* __restrict__ SRC,
-                                const double* __restrict__ prof, const Geo& g, const Sk& q, int tile, int TY,
-                                double deltaT) {
-  constexpr int NF = XY ? 7 : 12;
-  const int lane = threadIdx.x & 63;
+// wave 9: the split-Jacobian entries of the cross-tile neighbours, from their
+// summaries (along x the compact edge copy, along y the neighbour tile's row), into the halo columns of slot sig - 1.
+// Lane 16 d + c serves consumer c at step 4 m + d.  The entries of steps
+// 4 m .. 4 m + 2 go to LDS during step 4 m - 1, those of step 4 m + 3, whose
+// slot is still being read then, during step 4 m.
+template <bool FWD, class T>
+__device__ __forceinline__ void pipe_halo_coef(PipeLds<T>& L, const T* __restrict__ S, const T* __restrict__ E,
+                                               const double* __restrict__ prof, const Geo& g, const Sk& q, int tile,
+                                               int TX, int TY) {
+  static_assert(PIPE_SLOTS == 4, "four steps of 16 lanes");
+  const int lane = threadIdx.x & 63, c = lane & 15, d4 = lane >> 4;
+  const HaloLane<FWD> h(c >> 3, c & 7, g, TX, TY);
   const int nsteps = q.nsteps;
   const long nf = q.nsk;
-  const long row0 = (long)tile * nsteps * 64 + lane;
-  // metric of the lane's j (clamped for columns outside the domain)
-  const int j = min(2 + TY * TJ + (lane >> 3), g.ny);
-  const T nx = T(pf(prof, g.Ym, SET_C, 1, j)), ny_ = T(pf(prof, g.Ym, SET_C, 5, j)),
-          nz_ = T(pf(prof, g.Ym, SET_C, 9, j));
-  // fields: XY: P beta rho UX LX UY LY;
-  //         z:  SRC0..4 P beta rho LX LY UZ LZ
-  auto field = [&](int f) -> const T* {
-    if (XY) return S + (long)(f < 3 ? G_P + f : G_UX + (f - 3)) * nf;
-    if (f < 5) return SRC + (long)f * nf;
-    if (f < 8) return S + (long)(G_P + (f - 5)) * nf;
-    constexpr int zf[4] = {G_LX, G_LY, G_UZ, G_LZ};
-    return S + (long)zf[f - 8] * nf;
-  };
-  Slots<QS, NF, T> buf;
-  auto issue = [&](int sig, int sl) {
-    const int sc = min(sig, nsteps - 1);
-    const long c = row0 + (long)(FWD ? sc : nsteps - 1 - sc) * 64;
-    T d[NF];
-#pragma unroll
-    for (int f = 0; f < NF; f++) d[f] = field(f)[c];
-    buf.put(sl, d);
-  };
-  auto consume = [&](int sig, int sl) {
-    if (sig >= nsteps) return;
-    T d[NF];
-    buf.get(sl, d);
-    const int s3 = sig % 3;
-    if constexpr (XY) {
-      const T Tc = over_rho(d[0], d[2]);
-      T pdx, p51x, pdy, p51y;
-      split_pd_p51(nx, d[3], d[1], d[2], &pdx, &p51x);
-      split_pd_p51(ny_, d[5], d[1], d[2], &pdy, &p51y);
-      coef_store(L.xc[s3], lane, diag_coef<0, FWD>(d[0], Tc, d[1], d[3], d[4], pdx, p51x, nx));
-      coef_store(L.yc[s3], lane, diag_coef<1, FWD>(d[0], Tc, d[1], d[5], d[6], pdy, p51y, ny_));
-    } else {
-      // d: SRC0..4, P, beta, rho, LX, LY, UZ, LZ
-      T d11, d22, d51;
-      diag_dinv(d[6], d[7], d[8], d[9], d[11], g.dXI, g.dET, g.dZT, deltaT, &d11, &d22, &d51);
-      L.own[s3][PO_D11][lane] = d11;
-      L.own[s3][PO_D22][lane] = d22;
-      L.own[s3][PO_D51][lane] = d51;
-#pragma unroll
-      for (int f = 0; f < 5; f++) L.own[s3][PO_M + f][lane] = d[f];
-      const T Tc = over_rho(d[5], d[7]);
-      T pdz, p51z;
-      split_pd_p51(nz_, d[10], d[6], d[7], &pdz, &p51z);
-      const SplitCoefT<T> z = diag_coef<2, FWD>(d[5], Tc, d[6], d[10], d[11], pdz, p51z, nz_);
-      L.own[s3][PO_Z + 0][lane] = z.c11;
-      L.own[s3][PO_Z + 1][lane] = z.c1q;
-      L.own[s3][PO_Z + 2][lane] = z.c22;
-      L.own[s3][PO_Z + 3][lane] = z.c5q;
-      L.own[s3][PO_Z + 4][lane] = z.pd;
-      L.own[s3][PO_Z + 5][lane] = z.p51;
-    }
-  };
-#pragma unroll
-  for (int k = 0; k < QS; k++) issue(k, k);
-  consume(0, 0);
-  issue(QS, 0);
-  lds_barrier();
-  pipe_loader_loop<QS>(nsteps, consume, issue);
-}
-
-// wave 3: the halo of the next step QD steps ahead.  There are 16 consumer
-// lanes of the compute wave: 0..7 on the x edge (b = c) and 8..15 on the y
-// edge (a = c - 8).  Each needs its remote cell's summary along the
-// direction (P beta rho U lam), which the prep pass wrote, and the remote
-// tile's NL/NR output (5 values), which may still be in flight.  Lane c of
-// the first 16 loads consumer c's five outputs; lane 16 + c loads its five
-// summary values, which reach lane c by cross-lane shuffles and become the
-// split-Jacobian entries before the outputs are polled, so that once they
-// arrive only their LDS stores stand between them and the barrier.
-template <bool FWD, int QD, class T>
-__device__ void pipe_halo_loader(PipeLds<T>& L, const T* __restrict__ S, const T* __restrict__ DST,
-                                 const double* __restrict__ prof, const Geo& g, const Sk& q, int tile, int TX,
-                                 int TY, int* err, long spin_limit) {
-  const int lane = threadIdx.x & 63;
-  const int cid = lane & 15, grp = lane >> 4;
-  const int nsteps = q.nsteps, Nz = q.Nz;
-  const long nf = q.nsk;
-  const int dir = cid < 8 ? 0 : 1;
-  const int idx = cid & 7;
-  const int a = dir == 0 ? (FWD ? 0 : TI - 1) : idx;  // consumer lane (a, b)
-  const int b = dir == 0 ? idx : (FWD ? 0 : TJ - 1);
-  const int i = 3 + TX * TI + a, j = 2 + TY * TJ + b;
-  const bool dom = dir == 0 ? (FWD ? i - 1 >= 3 : i + 1 <= g.gend) : (FWD ? j - 1 >= 2 : j + 1 <= g.ny);
-  const bool ok = i <= g.gend && j <= g.ny && dom;
-  const int off = FWD ? a + b : (TI - 1 - a) + (TJ - 1 - b);
-  const long sx = FWD ? (-(long)nsteps * 64 + 7 * 64 + 7) : ((long)nsteps * 64 - 7 * 64 - 7);
-  const long sy = FWD ? (-(long)q.nTI * nsteps * 64 + 7 * 64 + 56) : ((long)q.nTI * nsteps * 64 - 7 * 64 - 56);
-  const long own0 = (long)tile * nsteps * 64 + (a + 8 * b);
-  const long rem0 = own0 + (dir == 0 ? sx : sy);
+  static_assert(HO_SLOT == 64, "a step is 64 elements on in the edge copy and in the rows");
   // metric at the remote cell's j
-  const int jr = dir == 0 ? j : (FWD ? j - 1 : j + 1);
-  const T n = T(pf(prof, g.Ym, SET_C, dir == 0 ? 1 : 5, min(max(jr, 0), g.Ym - 1)));
-  const int dU = G_UX + 2 * dir;
-  auto live = [=](int sig) -> bool {
-    const int kk = sig - off;
-    return ok && kk >= 0 && kk < Nz && sig < nsteps;
-  };
-  const long rdiff = rem0 - own0;
-  auto cell = [=](int sig) -> long {
-    const int sc = min(sig, nsteps - 1);
-    return own0 + (live(sig) ? rdiff : 0L) + (long)(FWD ? sc : nsteps - 1 - sc) * 64;
-  };
-  // this lane's five fields: group 0 the outputs N0..N4, group 1 P beta rho
-  // U lam, groups 2 and 3 re-read group 1's (a uniform load count per step)
-  const bool outs = grp == 0;
+  const int j = 2 + TY * TJ + h.b;
+  const int jr = h.dir == 0 ? j : (FWD ? j - 1 : j + 1);
+  const T n = T(pf(prof, g.Ym, SET_C, h.dir == 0 ? 1 : 5, min(max(jr, 0), g.Ym - 1)));
+  // field f of the neighbour at its (forward) step p: fld[f] + p * 64; a
+  // consumer without a neighbour reads its own tile's
+  const int px = h.ok ? (FWD ? tile - 1 : tile + 1) : tile, py = h.ok ? (FWD ? tile - q.nTI : tile + q.nTI) : tile;
   const T* fld[5];
 #pragma unroll
-  for (int r = 0; r < 5; r++)
-    fld[r] = outs ? DST + (long)r * nf : (r < 3 ? S + (long)(G_P + r) * nf : S + (long)(dU + r - 3) * nf);
-  Slots<QD, 5, T> buf;
-  auto issue = [&](int sig, int sl) {
-    const long c = cell(sig);
-    T d[5];
+  for (int f = 0; f < 5; f++)
+    fld[f] = h.dir == 0 ? E + ho_at(q, px, FWD ? 0 : 1, 0) + 8 * f + h.idx
+                        : S + (long)(f < 3 ? G_P + f : G_UY + f - 3) * nf + sk_at(q, py, 0, (FWD ? 56 : 0) + h.idx);
+  T(*row)[72] = (h.dir == 0 ? L.xc : L.yc)[(d4 + 3) % PIPE_SLOTS];
+  T buf[2][5];
+  auto issue = [&](int s0, auto sl) {
+    // the consumer's step sig uses what the neighbour's walk has at sig + 7
+    const int sc = min(s0 + d4 + 7, nsteps - 1);
+    const long o = (long)(FWD ? sc : nsteps - 1 - sc) * 64;
 #pragma unroll
-    for (int r = 0; r < 5; r++) d[r] = ld_coherent(fld[r] + c);
-    buf.put(sl, d);
+    for (int f = 0; f < 5; f++) buf[sl][f] = ld_here(fld[f] + o);
   };
-  auto consume = [&](int sig, int sl) {
-    if (sig >= nsteps) return;
-    T d[5];
-    buf.get(sl, d);
-    const bool lv = live(sig);
-    const int sp = (sig + 2) % 3, np = (sig & 1) ^ 1;
-    // the remote summary to consumer lanes, and its split Jacobian
-    T v[5];
-#pragma unroll
-    for (int r = 0; r < 5; r++) v[r] = __shfl(d[r], cid + 16, 64);
-    if (outs && lv) {
-      const T Tc = over_rho(v[0], v[2]);
-      T pd, p51;
-      split_pd_p51(n, v[3], v[1], v[2], &pd, &p51);
-      if (dir == 0)
-        coef_store(L.xc[sp], 64 + idx, diag_coef<0, FWD>(v[0], Tc, v[1], v[3], v[4], pd, p51, n));
-      else
-        coef_store(L.yc[sp], 64 + idx, diag_coef<1, FWD>(v[0], Tc, v[1], v[3], v[4], pd, p51, n));
+  SplitCoefT<T> cf;
+  auto form = [&](auto sl) {
+    const T(&d)[5] = buf[sl];
+    const T rr = rcp_rho(d[2]);
+    cf = coef_of<FWD>(d[0], d[1], d[2], rr, over_rho(d[0], d[2], rr), d[3], d[4], n, h.dir == 0);
+  };
+  issue(0, Int<0>{});
+  issue(4, Int<1>{});
+  form(Int<0>{});
+  if (d4 < 3) coef_store(row, 64 + h.idx, cf);
+  lds_barrier();
+  int tau = 0;
+  cycle<8>([&](auto k) -> bool {
+    constexpr int K = decltype(k)::value % 4, B = decltype(k)::value / 4;
+    if constexpr (K == 0) {
+      if (d4 == 3) coef_store(row, 64 + h.idx, cf);
+      issue(tau + 8, Int<B>{});
+    } else if constexpr (K == 3) {
+      form(Int<1 - B>{});
+      if (d4 < 3) coef_store(row, 64 + h.idx, cf);
     }
-    bool pend = false;
-    if (outs && lv) {
-#pragma unroll
-      for (int r = 0; r < 5; r++) pend |= is_sentinel(d[r]);
-    }
+    lds_barrier();
+    return ++tau < nsteps;
+  });
+}
+
+// The 80 values a tile takes over per step (x edge, then y edge: 5 components
+// x 8 cells each): lane l has values l and, below lane 16, 64 + l.  p0, p1:
+// their producers' slots of step 0.
+template <bool FWD, class T>
+struct HaloValues {
+  int r0, r1;
+  bool two;
+  HaloLane<FWD> h0, h1;
+  T *p0, *p1;
+  __device__ __forceinline__ HaloValues(T* __restrict__ H, const Geo& g, const Sk& q, int tile, int TX, int TY, int lane)
+      : r0(lane < 40 ? lane : lane - 40),
+        r1(lane + 24),
+        two(lane < 16),
+        h0(lane < 40 ? 0 : 1, r0 & 7, g, TX, TY),
+        h1(1, r1 & 7, g, TX, TY) {
+    const int px = FWD ? tile - 1 : tile + 1, py = FWD ? tile - q.nTI : tile + q.nTI;
+    p0 = H + ho_at(q, h0.ok ? (h0.dir == 0 ? px : py) : tile, h0.dir, 0) + r0;
+    p1 = two ? H + ho_at(q, h1.ok ? py : tile, 1, 0) + r1 : p0;
+  }
+  __device__ __forceinline__ bool live0(int sig, const Sk& q) const { return h0.live(sig, q); }
+  __device__ __forceinline__ bool live1(int sig, const Sk& q) const { return two && h1.live(sig, q); }
+  // the consumer's step sig reads what the producer formed at its step sig + 7
+  __device__ __forceinline__ static long slot(int sig, const Sk& q) {
+    return (long)min(sig + 7, q.nsteps - 1) * HO_SLOT;
+  }
+};
+
+// waves 6 and 7 (odd): the cross-tile neighbours' outputs of every second
+// step, polled.  A coherent load takes about a microsecond, two steps' time,
+// so each wave has its next step's load in flight while the other takes its
+// own over.  Looking further ahead lengthens every hop instead: a tile that
+// finds a value missing waits, and so falls behind its upstream tiles until
+// its loads, issued that much earlier, succeed.
+template <bool FWD, class T>
+__device__ __forceinline__ void pipe_halo_poll(PipeLds<T>& L, T* __restrict__ H, const Geo& g, const Sk& q, int tile,
+                                               int TX, int TY, int odd, int* err, long spin_limit) {
+  const int lane = threadIdx.x & 63;
+  const int nsteps = q.nsteps;
+  const HaloValues<FWD, T> hv(H, g, q, tile, TX, TY, lane);
+  T *p0 = hv.p0, *p1 = hv.p1;
+  // step sig's values go to the half of N that step sig - 1 fills
+  T* l0 = &L.N[odd ^ 1][min(hv.r0 >> 3, 4)][(hv.h0.dir == 0 ? 64 : 72) + hv.h0.idx];
+  T* l1 = &L.N[odd ^ 1][min(hv.r1 >> 3, 4)][72 + hv.h1.idx];
+  T v0, v1;
+  auto issue = [&](int sig) {
+    const long s = hv.slot(sig, q);
+    v0 = ld_coherent(p0 + s);
+    v1 = ld_coherent(p1 + s);  // a lane without a second value reads its first again
+  };
+  auto consume = [&](int sig) {
+    const bool lv0 = hv.live0(sig, q), lv1 = hv.live1(sig, q);
+    bool pend = (lv0 && is_sentinel(v0)) || (lv1 && is_sentinel(v1));
     long cnt = 0;
     while (__any(pend)) {
       // one memory round trip per poll: the pending outputs and the error
       // flag (set by a tile that gave up) are loaded together
       const int e = __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (pend) {
-        const long c = cell(sig);
-        pend = false;
-#pragma unroll
-        for (int r = 0; r < 5; r++) {
-          d[r] = ld_coherent(fld[r] + c);
-          pend |= is_sentinel(d[r]);
-        }
-      }
+      issue(sig);
+      pend = (lv0 && is_sentinel(v0)) || (lv1 && is_sentinel(v1));
       if (__builtin_amdgcn_readfirstlane(e) != 0 || ++cnt > spin_limit) {
         if (lane == 0) __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         break;
       }
     }
-    if (outs && lv) {
-#pragma unroll
-      for (int w = 0; w < 5; w++) L.N[np][w][(dir == 0 ? 64 : 72) + idx] = d[w];
-    }
+    if (lv0) *l0 = v0;
+    if (lv1) *l1 = v1;
   };
-#pragma unroll
-  for (int k = 0; k < QD; k++) issue(k, k);
-  consume(0, 0);
-  issue(QD, 0);
-  lds_barrier();
-  pipe_loader_loop<QD>(nsteps, consume, issue);
+  issue(odd);
+  // step sig is taken over during step sig - 1 (step 0 before the first);
+  // `left` barriers remain of the nsteps + 1 every wave passes
+  int left = nsteps + 1, sig = odd;
+  if (odd) {
+    lds_barrier();
+    left--;
+  }
+  for (;;) {
+    consume(sig);  // past the last step no value is live
+    sig += 2;
+    issue(sig);
+    lds_barrier();
+    if (--left == 0) break;
+    lds_barrier();
+    if (--left == 0) break;
+  }
 }
 
-template <bool FWD, int QS, int QD, class T>
-__global__ void __launch_bounds__(256) k_sweep_pipe(const T* __restrict__ S, T* __restrict__ SRC,
-                                                    T* __restrict__ DST, T* __restrict__ AUX,
-                                                    const double* __restrict__ prof, Geo g, Sk q,
-                                                    const int* __restrict__ order, int* __restrict__ sync,
-                                                    long spin_limit, double deltaT) {
-  // arrays in sweep order (Sk); S holds the DiagField summary
-  // FWD: SRC = MR, DST = NL   (NL = D^-1 (MR - L)); seeds the NR (AUX) sentinels
-  // BWD: SRC = NL, DST = NR   (NR = NL - D^-1 U); re-seeds the NL sentinels
-  __shared__ PipeLds<T> L;
+// wave 8: writes the outputs of the step before the one being computed to
+// their rows of DST (from the LDS half that the compute waves fill again only
+// after the next barrier) and sets the hand-off slots that waves 6, 7 have read
+// back to the sentinel.  It waits for no load, so these stores delay nobody:
+// stores and loads share one counter, and a wave that waits for a load waits
+// for its earlier stores too.
+template <bool FWD, class T>
+__device__ __forceinline__ void pipe_writer(PipeLds<T>& L, T* __restrict__ DST, T* __restrict__ H, const Geo& g,
+                                            const Sk& q, int tile, int TX, int TY) {
+  const int lane = threadIdx.x & 63;
+  const int a = lane & 7, b = lane >> 3;
+  const int nsteps = q.nsteps;
+  const long nf = q.nsk, row0 = (long)tile * nsteps * 64;
+  const bool col = 3 + TX * TI + a <= g.gend && 2 + TY * TJ + b <= g.ny;
+  const int off = FWD ? a + b : (TI - 1 - a) + (TJ - 1 - b);
+  const T sv = sentinel_value<T>();
+  const HaloValues<FWD, T> hv(H, g, q, tile, TX, TY, lane);
+  auto store_out = [&](int s, auto half) {
+    const int kk = s - off;
+    if (col && kk >= 0 && kk < q.Nz) {
+      T* r = DST + row0 + (long)(FWD ? s : nsteps - 1 - s) * 64;
+#pragma unroll
+      for (int v = 0; v < 5; v++) (r + (long)v * nf)[lane] = L.N[half][v][lane];
+    }
+  };
+  lds_barrier();
+  int tau = 0;
+  cycle<2>([&](auto k) -> bool {
+    store_out(tau - 1, Int<1 - decltype(k)::value>{});
+    const long s = hv.slot(tau, q);
+    if (hv.live0(tau, q)) st_coherent(hv.p0 + s, sv);
+    if (hv.live1(tau, q)) st_coherent(hv.p1 + s, sv);
+    lds_barrier();
+    return ++tau < nsteps;
+  });
+  if (nsteps & 1)
+    store_out(nsteps - 1, Int<0>{});
+  else
+    store_out(nsteps - 1, Int<1>{});
+}
+
+template <bool FWD, bool FD, class T>
+__device__ __forceinline__ void pipe_tile(PipeLds<T>& L, const T* __restrict__ S, const T* __restrict__ SRC,
+                                          T* __restrict__ DST, T* __restrict__ H, const T* __restrict__ E,
+                                          const double* __restrict__ prof, const Geo& g, const Sk& q, int tile,
+                                          int* err, long spin_limit, double deltaT) {
+  const int TX = tile % q.nTI, TY = tile / q.nTI;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  switch (wave) {
+    case 4:
+      __builtin_amdgcn_s_setprio(3);  // the step waits for these four
+      pipe_compute<FWD, FD, true>(L, H, g, q, tile, TX, TY);
+      break;
+    case 5:
+      __builtin_amdgcn_s_setprio(3);
+      pipe_compute<FWD, FD, false>(L, H, g, q, tile, TX, TY);
+      break;
+    case 6:
+    case 7:
+      __builtin_amdgcn_s_setprio(3);
+      pipe_halo_poll<FWD>(L, H, g, q, tile, TX, TY, wave - 6, err, spin_limit);
+      break;
+    case 8: pipe_writer<FWD>(L, DST, H, g, q, tile, TX, TY); break;
+    case 9: pipe_halo_coef<FWD>(L, S, E, prof, g, q, tile, TX, TY); break;
+    default: pipe_loader<FWD, FD>(L, S, SRC, prof, g, q, tile, TY, wave, deltaT); break;
+  }
+}
+
+template <bool FWD, class T>
+__global__ void __launch_bounds__(PIPE_THREADS) k_sweep_pipe(const T* __restrict__ S, const T* __restrict__ SRC,
+                                                             T* __restrict__ DST, T* __restrict__ H,
+                                                             const T* __restrict__ E,
+                                                             const double* __restrict__ prof, Geo g, Sk q,
+                                                             const int* __restrict__ order, int* __restrict__ sync,
+                                                             long spin_limit, double deltaT) {
+  // arrays in sweep order (Sk); S holds the DiagField summary, E its copy of
+  // the x edges, H the hand-off slots
+  // FWD: SRC = MR, DST = NL   (NL = D^-1 (MR - L))
+  // BWD: SRC = NL, DST = NR   (NR = NL - D^-1 U)
+  __shared__ PipeLds<T> L;
   if (threadIdx.x == 0) L.ticket = atomicAdd(sync, 1);
   __syncthreads();
-  const int t = L.ticket;
+  // the ticket is the same for all lanes: rows and slots get scalar addresses
+  const int t = __builtin_amdgcn_readfirstlane(L.ticket);
   if (t >= q.ntiles) return;
   const int tile = order[FWD ? t : q.ntiles - 1 - t];
-  const int TX = tile % q.nTI, TY = tile / q.nTI;
-  if (wave == 0) {
-    // the kernel arguments make this choice uniform: one scalar branch
-    if constexpr (std::is_same<T, double>::value) {
-      if (g.rXI != 0.0 && g.rET != 0.0 && g.rZT != 0.0)
-        pipe_compute<FWD, true>(L, SRC, DST, AUX, g, q, tile, TX, TY);
-      else
-        pipe_compute<FWD, false>(L, SRC, DST, AUX, g, q, tile, TX, TY);
-    } else {
-      pipe_compute<FWD, false>(L, SRC, DST, AUX, g, q, tile, TX, TY);
+  // the kernel arguments make this choice uniform: one scalar branch
+  if constexpr (std::is_same<T, double>::value) {
+    if (g.fast_div) {
+      pipe_tile<FWD, true>(L, S, SRC, DST, H, E, prof, g, q, tile, sync + 1, spin_limit, deltaT);
+      return;
     }
-  } else if (wave == 1) {
-    pipe_own_loader<FWD, true, QS>(L, S, SRC, prof, g, q, tile, TY, deltaT);
-  } else if (wave == 2) {
-    pipe_own_loader<FWD, false, QS>(L, S, SRC, prof, g, q, tile, TY, deltaT);
-  } else {
-    pipe_halo_loader<FWD, QD>(L, S, DST, prof, g, q, tile, TX, TY, sync + 1, spin_limit);
   }
+  pipe_tile<FWD, false>(L, S, SRC, DST, H, E, prof, g, q, tile, sync + 1, spin_limit, deltaT);
+}
+
+// every hand-off slot set to the sentinel: a new buffer, or after a sweep that
+// gave up (a sweep that ends leaves them so); two steps of a tile per block
+template <class T>
+__global__ void __launch_bounds__(256) k_seed_hand_off(T* __restrict__ H, Sk q) {
+  const int dir = (threadIdx.x >> 6) & 1, s = blockIdx.x * 2 + (threadIdx.x >> 7);
+  if (s < q.nsteps) H[ho_at(q, blockIdx.y, dir, s) + (threadIdx.x & 63)] = sentinel_value<T>();
 }
 
 // ---------------------------------------------------------------------------
@@ -2658,13 +2825,18 @@ int sweep_tiles(const Geo& g, int* nTI, int* nTJ) {
 
 long sweep_field_elems(const Geo& g) { return sweep_layout(g).nsk; }
 
+long sweep_buffer_elems(const Geo& g) {
+  const Sk q = sweep_layout(g);
+  return (G_N + 15) * q.nsk + 2 * ho_at(q, q.ntiles, 0, 0);
+}
+
 long sweep_update_blocks(const Geo& g) {
   Sk q = sweep_layout(g);
   return (long)((q.nsteps + 3) / 4) * q.ntiles;
 }
 
-// Sbuf holds G_N summary fields, then MR, NL, NR (5 each) in sweep order, as
-// T; a float layout uses the first half of the buffer
+// Sbuf holds G_N summary fields, MR, NL, NR (5 each) in sweep order, then the
+// hand-off slots and the x edges' summary, as T; a float layout uses the first half of the buffer
 template <class T>
 static void sweeps_t(hipStream_t st, double* Ui, const double* MR, double* Sbuf, const double* prof, const Geo& g,
                      double deltaT, int n_sweeps, const int* order, int* sync, double* partial, double* er_dev,
@@ -2674,12 +2846,14 @@ static void sweeps_t(hipStream_t st, double* Ui, const double* MR, double* Sbuf,
   T* MRs = S + (long)G_N * q.nsk;
   T* NLs = MRs + 5 * q.nsk;
   T* NRs = NLs + 5 * q.nsk;
+  T* H = NRs + 5 * q.nsk;
+  T* E = H + ho_at(q, q.ntiles, 0, 0);
   if (rin)
     hipLaunchKernelGGL(k_sweep_prep_rhs<T>, dim3((q.nsteps + PR - 1) / PR, q.ntiles), dim3(PR_THREADS), 0, st, Ui, *rin,
-                       prof, S, MRs, g, q, deltaT);
+                       prof, S, MRs, E, g, q, deltaT);
   else
     hipLaunchKernelGGL(k_sweep_prep<T>, dim3((q.nsteps + PC - 1) / PC, q.ntiles), dim3(256), 0, st, Ui, MR, prof, S,
-                       MRs, g, q);
+                       MRs, E, g, q);
   if (marks) (void)hipEventRecord(marks[0], st);
   const int nt = q.ntiles;
   for (int sweep = 0; sweep < n_sweeps; sweep++) {
@@ -2691,8 +2865,8 @@ static void sweeps_t(hipStream_t st, double* Ui, const double* MR, double* Sbuf,
                            spin_limit, deltaT);
     }
     if (pipelined)
-      hipLaunchKernelGGL((k_sweep_pipe<true, PIPE_QS, PIPE_QD, T>), dim3(nt), dim3(256), 0, st, S, MRs, NLs, NRs,
-                         prof, g, q, order, sync, spin_limit, deltaT);
+      hipLaunchKernelGGL((k_sweep_pipe<true, T>), dim3(nt), dim3(PIPE_THREADS), 0, st, S, MRs, NLs, H,
+                         E, prof, g, q, order, sync, spin_limit, deltaT);
     if (marks) (void)hipEventRecord(marks[2 + 3 * sweep], st);
     if constexpr (std::is_same<T, double>::value) {
       if (!pipelined)
@@ -2700,8 +2874,8 @@ static void sweeps_t(hipStream_t st, double* Ui, const double* MR, double* Sbuf,
                            sync + nt + 2, spin_limit, deltaT);
     }
     if (pipelined)
-      hipLaunchKernelGGL((k_sweep_pipe<false, PIPE_QS, PIPE_QD, T>), dim3(nt), dim3(256), 0, st, S, NLs, NRs, NRs,
-                         prof, g, q, order, sync + nt + 2, spin_limit, deltaT);
+      hipLaunchKernelGGL((k_sweep_pipe<false, T>), dim3(nt), dim3(PIPE_THREADS), 0, st, S, NLs, NRs, H,
+                         E, prof, g, q, order, sync + nt + 2, spin_limit, deltaT);
     if (marks) (void)hipEventRecord(marks[3 + 3 * sweep], st);
   }
   // primitive update reading NR from the sweep order
@@ -2714,8 +2888,8 @@ static void sweeps_t(hipStream_t st, double* Ui, const double* MR, double* Sbuf,
 template <class T>
 static void seed_hand_off_t(hipStream_t st, double* Sbuf, const Geo& g) {
   Sk q = sweep_layout(g);
-  T* NLs = reinterpret_cast<T*>(Sbuf) + (long)(G_N + 5) * q.nsk;
-  hipLaunchKernelGGL(k_seed_hand_off<T>, dim3((q.nsteps + 3) / 4, q.ntiles), dim3(256), 0, st, NLs, q);
+  T* H = reinterpret_cast<T*>(Sbuf) + (long)(G_N + 15) * q.nsk;
+  hipLaunchKernelGGL(k_seed_hand_off<T>, dim3((q.nsteps + 1) / 2, q.ntiles), dim3(256), 0, st, H, q);
 }
 
 void launch_seed_hand_off(hipStream_t st, double* Sbuf, const Geo& g, bool fp32) {
@@ -2723,6 +2897,12 @@ void launch_seed_hand_off(hipStream_t st, double* Sbuf, const Geo& g, bool fp32)
     seed_hand_off_t<float>(st, Sbuf, g);
   else
     seed_hand_off_t<double>(st, Sbuf, g);
+}
+
+void launch_seed_tiles(hipStream_t st, double* Sbuf, const Geo& g) {
+  Sk q = sweep_layout(g);
+  hipLaunchKernelGGL(k_seed_tiles, dim3((q.nsteps + 3) / 4, q.ntiles), dim3(256), 0, st, Sbuf + (long)(G_N + 5) * q.nsk,
+                     q);
 }
 
 void launch_sweeps(hipStream_t st, double* Ui, const double* MR, double* Sbuf, const double* prof, const Geo& g,

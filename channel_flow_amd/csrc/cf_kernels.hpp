@@ -40,6 +40,7 @@ void launch_rhs(hipStream_t st, const double* Ui, const double* Un, const double
                 const Geo& g, double deltaT, double f_drive);
 int sweep_tiles(const Geo& g, int* nTI, int* nTJ);
 long sweep_field_elems(const Geo& g);
+long sweep_buffer_elems(const Geo& g);  // doubles in Sbuf
 long sweep_update_blocks(const Geo& g);
 // inputs of the RHS, for the sweep pre-pass that forms MR itself (rin)
 struct RhsIn {
@@ -48,8 +49,7 @@ struct RhsIn {
 };
 // Persistent tiled sweeps (diagonal metrics): the summary pre-pass (forming MR
 // with the RHS when rin is given, else reading MR), n_sweeps forward/backward
-// pairs, then the primitive update of Ui and er.  Sbuf: G_N + 15 fields of
-// sweep_field_elems doubles.  marks (optional, 1 + 3 * n_sweeps events) are
+// pairs, then the primitive update of Ui and er.  Sbuf: sweep_buffer_elems doubles.  marks (optional, 1 + 3 * n_sweeps events) are
 // recorded after the pre-pass, then per sweep after the sync reset, the
 // forward and the backward sweep.  fp32: the sweep-order fields, D^-1, the
 // split Jacobians and the sweeps in float (pipelined schedule only); the RHS
@@ -60,7 +60,9 @@ void launch_sweeps(hipStream_t st, double* Ui, const double* MR, double* Sbuf, c
                    const RhsIn* rin = nullptr, bool fp32 = false);
 // NL and NR of the last sweep back in the natural layout
 void launch_sweep_outputs(hipStream_t st, const double* Sbuf, double* NL, double* NR, const Geo& g, bool fp32 = false);
-// the forward sweep's cross-tile NL slots in Sbuf set to the sentinel
+// the single-wave tiles' cross-tile NL slots in Sbuf set to the sentinel
+void launch_seed_tiles(hipStream_t st, double* Sbuf, const Geo& g);
+// the pipelined sweeps' hand-off slots in Sbuf set to the sentinel
 void launch_seed_hand_off(hipStream_t st, double* Sbuf, const Geo& g, bool fp32);
 
 void launch_sweeps_planes(hipStream_t st, const double* Ui, const double* MR, double* NL, double* NR,
