@@ -87,7 +87,8 @@ struct cf_ctx {
   int schedule = 0;       // 0: persistent tiles, 1: one hyperplane per launch
   int solver = 0;         // implicit part: 0 LU-SGS (Dual_time_stepping), 1 DPLUSGS
   int visc_schedule = 0;  // 0: fused viscous kernel, 1: three kernels through Pr/VS (allocated on first use)
-  long prof_gen = 0;  // metric uploads so far
+  long prof_gen = 0;        // metric uploads so far
+  bool prof_dirty = false;  // hprof holds values that were not uploaded (a refused metric)
   bool fp32 = false;      // CF_FP32_SWEEPS: LU-SGS sweeps and split Jacobians in float
   int guess_order = 0;    // initial iterate of cf_physical_step: 0 U^n, 1 linear, 2 quadratic extrapolation
   double* Uqq = nullptr;  // U^{n-2} (5 fields), kept while guess_order is 2 (allocated on first use)
@@ -142,6 +143,7 @@ struct cf_ctx {
   double* partial = nullptr;
   double* er_dev = nullptr;   // the norms, then the two sweep error flags
   double* er_host = nullptr;  // pinned copy of er_dev, read after each iteration
+  double* pin = nullptr;      // pinned buffer for small host arrays (PIN_ELEMS)
   double* stat = nullptr;  // running per-j sums of Statistic's mean profiles (7 * Ym)
   double* shear = nullptr; // wall values of Statistic's y-face viscous flux (2 * X_out * Z_out)
   // Shear_stress.dat: running sums SXYm[1], SXYm[ny] and the previous running
@@ -171,40 +173,79 @@ static int fail(cf_ctx* c, int code, const char* fmt, ...) {
     if (e_ != hipSuccess) return fail((c), CF_ERR_HIP, "%s: %s", #expr, hipGetErrorString(e_)); \
   } while (0)
 
+constexpr long PIN_ELEMS = 1L << 17;  // doubles of a context's pinned buffer (1 MB)
+
 static long host_elems(const cf_ctx* c) { return (long)c->g.Xnp * c->g.Ym * c->g.Zm; }
 
-// reference layout (Z_m pitch) <-> device layout (Zp pitch), one field
-static int h2d(cf_ctx* c, double* dst, const double* src) {
-  HIPCHK(c, hipMemcpy2DAsync(dst, (size_t)c->g.Zp * 8, src, (size_t)c->g.Zm * 8, (size_t)c->g.Zm * 8,
-                             (size_t)c->g.Xnp * c->g.Ym, hipMemcpyHostToDevice, c->stream));
-  return CF_OK;
-}
-static int d2h(cf_ctx* c, double* dst, const double* src) {
-  HIPCHK(c, hipMemcpy2DAsync(dst, (size_t)c->g.Zm * 8, src, (size_t)c->g.Zp * 8, (size_t)c->g.Zm * 8,
-                             (size_t)c->g.Xnp * c->g.Ym, hipMemcpyDeviceToHost, c->stream));
-  return CF_OK;
-}
-static int h2d_n(cf_ctx* c, double* dst, const double* const* src, int n) {
-  for (int v = 0; v < n; v++) {
-    if (!src[v]) return fail(c, CF_ERR_ARG, "null input array %d", v);
-    int r = h2d(c, dst + v * c->g.nf, src[v]);
-    if (r) return r;
-  }
-  return CF_OK;
-}
-static int d2h_n(cf_ctx* c, double* const* dst, const double* src, int n) {
-  for (int v = 0; v < n; v++) {
-    if (!dst[v]) continue;
-    int r = d2h(c, dst[v], src + v * c->g.nf);
-    if (r) return r;
-  }
-  return CF_OK;
-}
 static int sync(cf_ctx* c) {
   HIPCHK(c, hipStreamSynchronize(c->stream));
   HIPCHK(c, hipGetLastError());
   return CF_OK;
 }
+
+// Fields that a contiguous staging copy takes at once: the sweep buffer's
+// summary and MR part, which holds nothing between sweeps.  Every use is
+// ordered on the context's stream.
+static int stage_fields(const cf_ctx* c, long elems) {
+  return (int)std::min(16L, std::max(1L, cf::sweep_scratch_elems(c->g) / elems));
+}
+
+// n host fields of `elems` doubles each -> the staging copy, in the stream's
+// order.  Small ones go through pinned memory in one copy: a copy per field
+// costs more than the bytes.
+static int stage_in(cf_ctx* c, const double* const* src, int n, long elems) {
+  for (int v = 0; v < n; v++)
+    if (!src[v]) return fail(c, CF_ERR_ARG, "null input array %d", v);
+  if (n * elems <= PIN_ELEMS) {
+    if (int r = sync(c)) return r;  // the pinned buffer is free
+    for (int v = 0; v < n; v++) memcpy(c->pin + v * elems, src[v], elems * sizeof(double));
+    HIPCHK(c, hipMemcpyAsync(c->Sm, c->pin, n * elems * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    return CF_OK;
+  }
+  for (int v = 0; v < n; v++)
+    HIPCHK(c, hipMemcpyAsync(c->Sm + v * elems, src[v], elems * sizeof(double), hipMemcpyHostToDevice, c->stream));
+  return CF_OK;
+}
+
+// the staging copy -> n host fields (null ones are skipped); done on return
+static int stage_out(cf_ctx* c, double* const* dst, int n, long elems) {
+  if (n * elems <= PIN_ELEMS) {
+    HIPCHK(c, hipMemcpyAsync(c->pin, c->Sm, n * elems * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    if (int r = sync(c)) return r;
+    for (int v = 0; v < n; v++)
+      if (dst[v]) memcpy(dst[v], c->pin + v * elems, elems * sizeof(double));
+    return CF_OK;
+  }
+  for (int v = 0; v < n; v++)
+    if (dst[v])
+      HIPCHK(c, hipMemcpyAsync(dst[v], c->Sm + v * elems, elems * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  return sync(c);
+}
+
+// reference layout (Z_m pitch) <-> device layout (Zp pitch)
+static int h2d_n(cf_ctx* c, double* dst, const double* const* src, int n) {
+  const long elems = host_elems(c);
+  const int most = stage_fields(c, elems);
+  for (int v = 0; v < n; v += most) {
+    const int m = std::min(most, n - v);
+    if (int r = stage_in(c, src + v, m, elems)) return r;
+    cf::launch_rows_in(c->stream, c->Sm, dst + v * c->g.nf, m, c->g);
+    HIPCHK(c, hipGetLastError());
+  }
+  return CF_OK;
+}
+static int d2h_n(cf_ctx* c, double* const* dst, const double* src, int n) {
+  const long elems = host_elems(c);
+  const int most = stage_fields(c, elems);
+  for (int v = 0; v < n; v += most) {
+    const int m = std::min(most, n - v);
+    cf::launch_rows_out(c->stream, src + v * c->g.nf, c->Sm, m, c->g);
+    HIPCHK(c, hipGetLastError());
+    if (int r = stage_out(c, dst + v, m, elems)) return r;
+  }
+  return CF_OK;
+}
+static int h2d(cf_ctx* c, double* dst, const double* src) { return h2d_n(c, dst, &src, 1); }
 
 // ---------------------------------------------------------------------------
 // metric j-profiles: the reference metrics (Jacobian*.cpp) depend only on j.
@@ -233,6 +274,22 @@ static int ingest(cf_ctx* c, const double* A, int set, int comp, const char* nam
   const Geo& g = c->g;
   Region r = region_of(c, set, comp);
   double* prof = &c->hprof[(size_t)(set * 10 + comp) * g.Ym];
+  c->prof_dirty = true;
+  // one pass in memory order; the loop below names the element where it fails
+  // (and lets equal NaNs through)
+  bool same = true;
+  for (int i = r.i0; same && i <= r.i1; i++)
+    for (int j = r.j0; same && j <= r.j1; j++) {
+      const double v0 = A[((size_t)r.i0 * g.Ym + j) * g.Zm + r.k0];
+      const double* row = A + ((size_t)i * g.Ym + j) * g.Zm;
+      int differ = 0;
+      for (int k = r.k0; k <= r.k1; k++) differ |= !(row[k] == v0);
+      same = !differ;
+    }
+  if (same) {
+    for (int j = r.j0; j <= r.j1; j++) prof[j] = A[((size_t)r.i0 * g.Ym + j) * g.Zm + r.k0];
+    return CF_OK;
+  }
   for (int j = r.j0; j <= r.j1; j++) {
     double v0 = A[((size_t)r.i0 * g.Ym + j) * g.Zm + r.k0];
     for (int i = r.i0; i <= r.i1; i++)
@@ -248,6 +305,7 @@ static int ingest(cf_ctx* c, const double* A, int set, int comp, const char* nam
 
 static int upload_prof(cf_ctx* c) {
   c->prof_gen++;
+  c->prof_dirty = false;
   HIPCHK(c, hipMemcpyAsync(c->prof, c->hprof.data(), c->hprof.size() * 8, hipMemcpyHostToDevice, c->stream));
   cf::launch_flux_tables(c->stream, c->prof, c->g);
   HIPCHK(c, hipGetLastError());
@@ -342,13 +400,14 @@ extern "C" int cf_create(const cf_params* p, cf_ctx** out) {
   if (hipMalloc(&c->partial, (size_t)nb * 5 * sizeof(double)) != hipSuccess) return bail(CF_ERR_HIP);
   if (hipMalloc(&c->er_dev, 8 * sizeof(double)) != hipSuccess) return bail(CF_ERR_HIP);
   if (hipHostMalloc(&c->er_host, 8 * sizeof(double), hipHostMallocDefault) != hipSuccess) return bail(CF_ERR_HIP);
+  if (hipHostMalloc(&c->pin, PIN_ELEMS * sizeof(double), hipHostMallocDefault) != hipSuccess) return bail(CF_ERR_HIP);
   if (hipMalloc(&c->stat, (size_t)7 * g.Ym * sizeof(double)) != hipSuccess) return bail(CF_ERR_HIP);
   if (hipMalloc(&c->shear, (size_t)2 * p->X_out * p->Z_out * sizeof(double)) != hipSuccess) return bail(CF_ERR_HIP);
   if (hipMemsetAsync(c->stat, 0, (size_t)7 * g.Ym * sizeof(double), c->stream) != hipSuccess) return bail(CF_ERR_HIP);
-  if (hipMalloc(&c->prof, (size_t)cf::PROF_ROWS * g.Ym * sizeof(double)) != hipSuccess) return bail(CF_ERR_HIP);
+  if (hipMalloc(&c->prof, (size_t)(cf::PROF_ROWS + 1) * g.Ym * sizeof(double)) != hipSuccess) return bail(CF_ERR_HIP);
   if (hipMalloc(&c->ypt, (size_t)g.Ym * sizeof(double)) != hipSuccess) return bail(CF_ERR_HIP);
   if (hipMemsetAsync(c->ypt, 0, (size_t)g.Ym * sizeof(double), c->stream) != hipSuccess) return bail(CF_ERR_HIP);
-  if (hipMemsetAsync(c->prof, 0, (size_t)cf::PROF_ROWS * g.Ym * sizeof(double), c->stream) != hipSuccess)
+  if (hipMemsetAsync(c->prof, 0, (size_t)(cf::PROF_ROWS + 1) * g.Ym * sizeof(double), c->stream) != hipSuccess)
     return bail(CF_ERR_HIP);
   if (hipStreamSynchronize(c->stream) != hipSuccess) return bail(CF_ERR_HIP);
   *out = c;
@@ -374,6 +433,7 @@ extern "C" void cf_destroy(cf_ctx* c) {
   if (c->py) (void)hipFree(c->py);
   if (c->sync) (void)hipFree(c->sync);
   if (c->er_host) (void)hipHostFree(c->er_host);
+  if (c->pin) (void)hipHostFree(c->pin);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
 }
@@ -982,38 +1042,35 @@ extern "C" int cf_rk3nodt(cf_ctx* c, int RK, double deltaT, double er[5], double
 // ---------------------------------------------------------------------------
 // device-resident path
 // ---------------------------------------------------------------------------
-// interior Q [X_out][Y_out][Z_out] -> U = Q/J in the device layout
-static int upload_Q(cf_ctx* c, double* dst, const double* const Q[5]) {
-  const Geo& g = c->g;
-  const double* Jp = &c->hprof[0];
-  std::vector<double> buf((size_t)g.nf, 0.0);
-  size_t X = c->p.X_out, Y = c->p.Y_out, Z = c->p.Z_out;
-  for (int v = 0; v < 5; v++) {
-    if (!Q[v]) return fail(c, CF_ERR_ARG, "null state array %d", v);
-    std::fill(buf.begin(), buf.end(), 0.0);
-    for (size_t i = 0; i < X; i++)
-      for (size_t j = 0; j < Y; j++)
-        for (size_t k = 0; k < Z; k++)
-          buf[(i + 3) * g.plane + (j + 2) * g.Zp + (k + 2)] = Q[v][(i * Y + j) * Z + k] / Jp[j + 2];
-    HIPCHK(c, hipMemcpy(dst + v * g.nf, buf.data(), (size_t)g.nf * 8, hipMemcpyHostToDevice));
-  }
+// the cell J by j on the device, as the host has it
+static int device_J(cf_ctx* c, const double** J) {
+  *J = c->prof;
+  if (!c->prof_dirty) return CF_OK;
+  *J = c->prof + (size_t)cf::PROF_ROWS * c->g.Ym;
+  HIPCHK(c, hipMemcpyAsync(c->prof + (size_t)cf::PROF_ROWS * c->g.Ym, c->hprof.data(), c->g.Ym * sizeof(double),
+                           hipMemcpyHostToDevice, c->stream));
   return CF_OK;
 }
 
+static long interior_elems(const cf_ctx* c) { return (long)c->p.X_out * c->p.Y_out * c->p.Z_out; }
+
+// interior Q [X_out][Y_out][Z_out] -> U = Q/J in the device layout
+static int upload_Q(cf_ctx* c, double* dst, const double* const Q[5]) {
+  for (int v = 0; v < 5; v++)
+    if (!Q[v]) return fail(c, CF_ERR_ARG, "null state array %d", v);
+  const double* J;
+  int r;
+  if ((r = device_J(c, &J)) || (r = stage_in(c, Q, 5, interior_elems(c)))) return r;
+  cf::launch_q_in(c->stream, c->Sm, J, dst, c->g);
+  return sync(c);
+}
+
 static int download_Q(cf_ctx* c, double* const Q[5], const double* src) {
-  const Geo& g = c->g;
-  const double* Jp = &c->hprof[0];
-  std::vector<double> buf((size_t)g.nf);
-  size_t X = c->p.X_out, Y = c->p.Y_out, Z = c->p.Z_out;
-  for (int v = 0; v < 5; v++) {
-    if (!Q[v]) continue;
-    HIPCHK(c, hipMemcpy(buf.data(), src + v * g.nf, (size_t)g.nf * 8, hipMemcpyDeviceToHost));
-    for (size_t i = 0; i < X; i++)
-      for (size_t j = 0; j < Y; j++)
-        for (size_t k = 0; k < Z; k++)
-          Q[v][(i * Y + j) * Z + k] = buf[(i + 3) * g.plane + (j + 2) * g.Zp + (k + 2)] * Jp[j + 2];
-  }
-  return CF_OK;
+  const double* J;
+  if (int r = device_J(c, &J)) return r;
+  cf::launch_q_out(c->stream, src, J, c->Sm, c->g);
+  HIPCHK(c, hipGetLastError());
+  return stage_out(c, Q, 5, interior_elems(c));
 }
 
 extern "C" int cf_load_state(cf_ctx* c, const double* const Qn[5], const double* const Qnm1[5]) {
@@ -1021,7 +1078,9 @@ extern "C" int cf_load_state(cf_ctx* c, const double* const Qn[5], const double*
   if (!c->have_metrics) return fail(c, CF_ERR_STATE, "metrics not set (cf_jacobian_all / cf_set_metrics)");
   int r;
   if ((r = sync(c))) return r;
-  if ((r = upload_Q(c, c->Un, Qn)) || (r = upload_Q(c, c->Uq, Qnm1)) || (r = upload_Q(c, c->Ui, Qn))) return r;
+  if ((r = upload_Q(c, c->Un, Qn)) || (r = upload_Q(c, c->Uq, Qnm1))) return r;
+  HIPCHK(c, hipMemcpyAsync(c->Ui, c->Un, (size_t)c->g.nf * 5 * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
+  if ((r = sync(c))) return r;
   for (int v = 0; v < 5; v++) c->E[v] = 0;
   c->have_state = true;
   c->uqq_valid = false;

@@ -8,6 +8,7 @@
 // j-profiles (they vary only with j, Jacobian*.cpp).
 #include "cf_kernels.hpp"
 
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -2480,10 +2481,79 @@ __global__ void __launch_bounds__(1024) k_reduce_partials(const double* __restri
 }
 
 // ---------------------------------------------------------------------------
+// host arrays <-> device fields through a contiguous staging copy.  A copy
+// between the host and rows of another pitch moves one row (Zm doubles) at a
+// time, about 0.15 ms each here; a contiguous copy runs at the link's rate
+// (18-30 GB/s from pageable memory) and these passes at HBM's.
+// ---------------------------------------------------------------------------
+// reference layout (rows of Zm) -> device rows of Zp, blockIdx.y the field;
+// the padding is left alone
+__global__ void __launch_bounds__(256) k_rows_in(const double* __restrict__ src, double* __restrict__ dst, Geo g,
+                                                 unsigned n) {
+  for (unsigned e = blockIdx.x * 256 + threadIdx.x; e < n; e += gridDim.x * 256) {
+    const unsigned row = e / (unsigned)g.Zm, k = e - row * (unsigned)g.Zm;
+    dst[blockIdx.y * g.nf + (long)row * g.Zp + k] = src[(long)blockIdx.y * n + e];
+  }
+}
+
+__global__ void __launch_bounds__(256) k_rows_out(const double* __restrict__ src, double* __restrict__ dst, Geo g,
+                                                  unsigned n) {
+  for (unsigned e = blockIdx.x * 256 + threadIdx.x; e < n; e += gridDim.x * 256) {
+    const unsigned row = e / (unsigned)g.Zm, k = e - row * (unsigned)g.Zm;
+    dst[(long)blockIdx.y * n + e] = src[blockIdx.y * g.nf + (long)row * g.Zp + k];
+  }
+}
+
+// interior Q [X][Y][Z] -> U = Q / J in the device layout, zero elsewhere
+__global__ void __launch_bounds__(256) k_q_in(const double* __restrict__ Q, const double* __restrict__ J,
+                                              double* __restrict__ U, Geo g) {
+  const int k = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * 4 + threadIdx.y, i = blockIdx.z;
+  if (k >= g.Zp || j >= g.Ym) return;
+  const int X = g.gend - 2, Y = g.ny - 1, Z = g.nz - 1;
+  const bool in = i >= 3 && i <= g.gend && j >= 2 && j <= g.ny && k >= 2 && k <= g.nz;
+  const long c = at(g, i, j, k), e = ((long)(i - 3) * Y + (j - 2)) * Z + (k - 2), n = (long)X * Y * Z;
+#pragma unroll
+  for (int v = 0; v < 5; v++) U[v * g.nf + c] = in ? Q[v * n + e] / J[j] : 0.0;
+}
+
+// Q = U J of the interior, [X][Y][Z]
+__global__ void __launch_bounds__(256) k_q_out(const double* __restrict__ U, const double* __restrict__ J,
+                                               double* __restrict__ Q, Geo g) {
+  const int k = 2 + blockIdx.x * 64 + threadIdx.x, j = 2 + blockIdx.y * 4 + threadIdx.y, i = 3 + blockIdx.z;
+  if (k > g.nz || j > g.ny) return;
+  const int X = g.gend - 2, Y = g.ny - 1, Z = g.nz - 1;
+  const long c = at(g, i, j, k), e = ((long)(i - 3) * Y + (j - 2)) * Z + (k - 2), n = (long)X * Y * Z;
+#pragma unroll
+  for (int v = 0; v < 5; v++) Q[v * n + e] = U[v * g.nf + c] * J[j];
+}
+
+// ---------------------------------------------------------------------------
 // host-side launchers
 // ---------------------------------------------------------------------------
 static inline dim3 box_grid(int nk, int nj, int ni, dim3 blk) {
   return dim3((nk + blk.x - 1) / blk.x, (nj + blk.y - 1) / blk.y, ni);
+}
+
+static dim3 row_grid(long n, int fields) { return dim3((unsigned)std::min((n + 255) / 256, 4096L), fields); }
+
+void launch_rows_in(hipStream_t st, const double* src, double* dst, int fields, const Geo& g) {
+  const long n = (long)g.Xnp * g.Ym * g.Zm;
+  hipLaunchKernelGGL(k_rows_in, row_grid(n, fields), dim3(256), 0, st, src, dst, g, (unsigned)n);
+}
+
+void launch_rows_out(hipStream_t st, const double* src, double* dst, int fields, const Geo& g) {
+  const long n = (long)g.Xnp * g.Ym * g.Zm;
+  hipLaunchKernelGGL(k_rows_out, row_grid(n, fields), dim3(256), 0, st, src, dst, g, (unsigned)n);
+}
+
+void launch_q_in(hipStream_t st, const double* Q, const double* J, double* U, const Geo& g) {
+  dim3 blk(64, 4);
+  hipLaunchKernelGGL(k_q_in, box_grid(g.Zp, g.Ym, g.Xnp, blk), blk, 0, st, Q, J, U, g);
+}
+
+void launch_q_out(hipStream_t st, const double* U, const double* J, double* Q, const Geo& g) {
+  dim3 blk(64, 4);
+  hipLaunchKernelGGL(k_q_out, box_grid(g.nz - 1, g.ny - 1, g.gend - 2, blk), blk, 0, st, U, J, Q, g);
 }
 
 void launch_halo_bc(hipStream_t st, double* U, const double* prof, const Geo& g, int x_periodic) {
@@ -2824,6 +2894,9 @@ int sweep_tiles(const Geo& g, int* nTI, int* nTJ) {
 }
 
 long sweep_field_elems(const Geo& g) { return sweep_layout(g).nsk; }
+
+// (S + MR: rewritten by every sweep's pre-pass and read by no one after it)
+long sweep_scratch_elems(const Geo& g) { return (G_N + 5) * sweep_layout(g).nsk; }
 
 long sweep_buffer_elems(const Geo& g) {
   const Sk q = sweep_layout(g);

@@ -4,6 +4,13 @@
 
 namespace cf {
 
+// n contiguous reference-layout fields <-> n device fields (padded rows)
+void launch_rows_in(hipStream_t st, const double* src, double* dst, int fields, const Geo& g);
+void launch_rows_out(hipStream_t st, const double* src, double* dst, int fields, const Geo& g);
+// five contiguous interior fields Q [X][Y][Z] <-> U = Q / J (zero outside the
+// interior); J: the cell J by j, on the device
+void launch_q_in(hipStream_t st, const double* Q, const double* J, double* U, const Geo& g);
+void launch_q_out(hipStream_t st, const double* U, const double* J, double* Q, const Geo& g);
 void launch_halo_bc(hipStream_t st, double* U, const double* prof, const Geo& g, int x_periodic);
 void launch_flux(hipStream_t st, int dir, const double* U, const double* prof, double* F, const Geo& g);
 // rebuilds the derived flux rows of the profile buffer from its metric rows
@@ -40,7 +47,8 @@ void launch_rhs(hipStream_t st, const double* Ui, const double* Un, const double
                 const Geo& g, double deltaT, double f_drive);
 int sweep_tiles(const Geo& g, int* nTI, int* nTJ);
 long sweep_field_elems(const Geo& g);
-long sweep_buffer_elems(const Geo& g);  // doubles in Sbuf
+long sweep_buffer_elems(const Geo& g);   // doubles in Sbuf
+long sweep_scratch_elems(const Geo& g);  // doubles at its start that hold nothing between sweeps
 long sweep_update_blocks(const Geo& g);
 // inputs of the RHS, for the sweep pre-pass that forms MR itself (rin)
 struct RhsIn {
