@@ -138,7 +138,7 @@ __global__ void __launch_bounds__(256) k_flux_zs(const double* __restrict__ U, c
 }
 
 // Flux_X and Flux_Y with one thread per column of faces: lanes run along k
-// and each thread walks FC consecutive faces along the direction with cells
+// and each thread walks fc <= FC consecutive faces along the direction with cells
 // f-2 .. f+3 in registers, loading one new cell per face (and that one a
 // face ahead) where a thread per face loads up to six.  16 faces per
 // thread measured faster than 8 and equal to 32 at 256x192x256.
@@ -149,7 +149,7 @@ constexpr int FLUX_COL_WAVES = 3;
 
 template <int DIR>
 __global__ void __launch_bounds__(256, FLUX_COL_WAVES) k_flux_col(const double* __restrict__ U, const double* __restrict__ prof,
-                                                  double* __restrict__ F, Geo g) {
+                                                  double* __restrict__ F, Geo g, int fc) {
   static_assert(DIR == 0 || DIR == 1, "columns along x or y");
   // DIR 0: f in [2,gend] (i), a = j in [2,ny]; DIR 1: f in [1,ny] (j), a = i in [3,gend]
   const int k = 2 + blockIdx.x * blockDim.x + threadIdx.x;
@@ -160,7 +160,7 @@ __global__ void __launch_bounds__(256, FLUX_COL_WAVES) k_flux_col(const double* 
   const int i = DIR == 0 ? 0 : 3 + a, j = DIR == 0 ? 2 + a : 0;
   if (k > g.nz || (DIR == 0 ? j > g.ny : i > g.gend)) return;
   const int fmin = DIR == 0 ? 2 : 1, fmax = DIR == 0 ? g.gend : g.ny;
-  const int f0 = fmin + blockIdx.z * FC, f1 = min(f0 + FC - 1, fmax);
+  const int f0 = fmin + blockIdx.z * fc, f1 = min(f0 + fc - 1, fmax);
   // cells outside the array (j = -1 and j = ny + 3 next to the walls) are
   // clamped onto it; no recipe of those faces reads them
   const int cmax = DIR == 0 ? g.Xnp - 1 : g.Ym - 1;
@@ -334,14 +334,14 @@ template <int DIR>
 __global__ void __launch_bounds__(256, 2) k_flux_lim_col(const double* __restrict__ U,
                                                                          const double* __restrict__ Ep,
                                                                          const double* __restrict__ prof,
-                                                                         double* __restrict__ F, Geo g) {
+                                                                         double* __restrict__ F, Geo g, int fc) {
   static_assert(DIR == 0 || DIR == 1, "columns along x or y");
   const int k = 2 + blockIdx.x * blockDim.x + threadIdx.x;
   const int a = blockIdx.y * blockDim.y + (DIR == 0 ? wave_row() : (int)threadIdx.y);
   const int i = DIR == 0 ? 0 : 3 + a, j = DIR == 0 ? 2 + a : 0;
   if (k > g.nz || (DIR == 0 ? j > g.ny : i > g.gend)) return;
   const int fmin = DIR == 0 ? 2 : 1, fmax = DIR == 0 ? g.gend : g.ny;
-  const int f0 = fmin + blockIdx.z * FC, f1 = min(f0 + FC - 1, fmax);
+  const int f0 = fmin + blockIdx.z * fc, f1 = min(f0 + fc - 1, fmax);
   double u[5][6], jj[6];
 #pragma unroll
   for (int t = 0; t < 6; t++) lim_cell<DIR>(U, prof, g, f0 - 2 + t, i, j, k, u, jj, t);
@@ -664,7 +664,7 @@ __global__ void __launch_bounds__(256) k_visc_div(const double* __restrict__ VS,
 }
 
 // Fused viscous terms for diagonal metrics.  One block owns a VJ (j) x VK (k) tile of cells and a
-// run of VC planes in i.  The primitives of three consecutive planes, with a
+// run of vc planes in i (at most VC).  The primitives of three consecutive planes, with a
 // one-cell rim in j and k, live in LDS.  Each of the VJ*VK main threads
 // computes the x face above its cell and the y and z faces below it; a
 // fifth wave computes the tile's extra y-face row (j0+VJ) and z-face column
@@ -822,12 +822,12 @@ __device__ __forceinline__ void vface_z(const VLds& L, int sp, int s0, int sm, i
 
 __global__ void __launch_bounds__(VTHREADS) k_visc_fused(const double* __restrict__ U,
                                                          const double* __restrict__ prof, double* __restrict__ vF,
-                                                         Geo g, double invXI, double invET, double invZT,
+                                                         Geo g, int vc, double invXI, double invET, double invZT,
                                                          double inv4XI, double inv4ET, double inv4ZT) {
   __shared__ VLds L;
   const int tid = threadIdx.x;
   const int k0 = 2 + blockIdx.x * VK, j0 = 2 + blockIdx.y * VJ;
-  const int ib = 3 + blockIdx.z * VC, ie = min(ib + VC - 1, g.gend);
+  const int ib = 3 + blockIdx.z * vc, ie = min(ib + vc - 1, g.gend);
   const bool main_t = tid < VJ * VK;
   const int ty = main_t ? tid / VK : 0, tx = main_t ? tid % VK : 0;
   const int j = j0 + ty, k = k0 + tx;
@@ -2597,29 +2597,48 @@ void launch_flux_tables(hipStream_t st, double* prof, const Geo& g) {
   hipLaunchKernelGGL(k_flux_tables, dim3((24 * g.Ym + 127) / 128), dim3(128), 0, st, prof, g);
 }
 
+// Faces per thread of the column kernels: FC, halved until `rows` waves times
+// the runs of a column of nf faces fill the chip's 1024 SIMDs with six waves
+// each.  A run loads six cells before its first face, but with few waves the
+// time is that of one run, face after face.  Flux_X / Flux_Y: 64^3 38 / 38 us
+// with 16 faces, 16 / 16 with 1 (4160 waves); 128x96x128 62 / 60 us with 16,
+// 48 / 50 with 4 (6336); 256x192x256 438 / 434 us with 1, 322 / 329 with 16
+// (13056).
+static int flux_run(long rows, int nf) {
+  int fc = FC;
+  while (fc > 1 && rows * ((nf + fc - 1) / fc) < 6144) fc /= 2;
+  return fc;
+}
+
 void launch_flux(hipStream_t st, int dir, const double* U, const double* prof, double* F, const Geo& g) {
   dim3 blk(64, 4);
-  if (dir == 0)
-    hipLaunchKernelGGL(k_flux_col<0>, box_grid(g.nz - 1, g.ny - 1, (g.gend - 1 + FC - 1) / FC, blk), blk, 0, st, U,
-                       prof, F, g);
-  else if (dir == 1)
-    hipLaunchKernelGGL(k_flux_col<1>, box_grid(g.nz - 1, g.gend - 2, (g.ny + FC - 1) / FC, blk), blk, 0, st, U, prof,
-                       F, g);
-  else
+  if (dir == 2) {
     hipLaunchKernelGGL(k_flux_zs<2>, box_grid(g.nz, g.ny - 1, g.gend - 2, blk), blk, 0, st, U, prof, F, g);
+    return;
+  }
+  const int nr = dir == 0 ? g.ny - 1 : g.gend - 2, nf = dir == 0 ? g.gend - 1 : g.ny;
+  const int fc = flux_run((long)((g.nz - 1 + 63) / 64) * nr, nf);
+  const dim3 gr = box_grid(g.nz - 1, nr, (nf + fc - 1) / fc, blk);
+  if (dir == 0)
+    hipLaunchKernelGGL(k_flux_col<0>, gr, blk, 0, st, U, prof, F, g, fc);
+  else
+    hipLaunchKernelGGL(k_flux_col<1>, gr, blk, 0, st, U, prof, F, g, fc);
 }
 
 void launch_flux_limiter(hipStream_t st, int dir, const double* U, const double* Ep, const double* prof, double* F,
                          const Geo& g) {
   dim3 blk(64, 4);
-  if (dir == 0)
-    hipLaunchKernelGGL(k_flux_lim_col<0>, box_grid(g.nz - 1, g.ny - 1, (g.gend - 1 + FC - 1) / FC, blk), blk, 0, st, U,
-                       Ep, prof, F, g);
-  else if (dir == 1)
-    hipLaunchKernelGGL(k_flux_lim_col<1>, box_grid(g.nz - 1, g.gend - 2, (g.ny + FC - 1) / FC, blk), blk, 0, st, U, Ep,
-                       prof, F, g);
-  else
+  if (dir == 2) {
     hipLaunchKernelGGL(k_flux_lim<2>, box_grid(g.nz, g.ny - 1, g.gend - 2, blk), blk, 0, st, U, Ep, prof, F, g);
+    return;
+  }
+  const int nr = dir == 0 ? g.ny - 1 : g.gend - 2, nf = dir == 0 ? g.gend - 1 : g.ny;
+  const int fc = flux_run((long)((g.nz - 1 + 63) / 64) * nr, nf);
+  const dim3 gr = box_grid(g.nz - 1, nr, (nf + fc - 1) / fc, blk);
+  if (dir == 0)
+    hipLaunchKernelGGL(k_flux_lim_col<0>, gr, blk, 0, st, U, Ep, prof, F, g, fc);
+  else
+    hipLaunchKernelGGL(k_flux_lim_col<1>, gr, blk, 0, st, U, Ep, prof, F, g, fc);
 }
 
 void launch_filter(hipStream_t st, const double* U, const double* prof, const double* Yp, double* W, double crit,
@@ -2664,8 +2683,15 @@ void launch_viscous(hipStream_t st, const double* U, const double* prof, double*
   double invXI = 1. / (g.dXI), invET = 1. / (g.dET), invZT = 1. / (g.dZT);
   double inv4XI = 1. / (4 * g.dXI), inv4ET = 1. / (4 * g.dET), inv4ZT = 1. / (4 * g.dZT);
   if (fused_viscous) {
-    dim3 gr((g.nz - 1 + VK - 1) / VK, (g.ny - 1 + VJ - 1) / VJ, (g.gend - 2 + VC - 1) / VC);
-    hipLaunchKernelGGL(k_visc_fused, gr, dim3(VTHREADS), 0, st, U, prof, vF, g, invXI, invET, invZT, inv4XI, inv4ET,
+    // planes per block: VC, halved until two blocks per CU are there.  64^3: 53
+    // us with 16 planes, 21 with 2 (512 blocks); 16x12x16: 48 and 10 (1 plane);
+    // 128x96x128: 85 with 16, 72 with 8 (768 blocks), 88 with 4; 256x192x256:
+    // 542 with 16, 605 with 4.
+    const long tiles = (long)((g.nz - 1 + VK - 1) / VK) * ((g.ny - 1 + VJ - 1) / VJ);
+    int vc = VC;
+    while (vc > 1 && tiles * ((g.gend - 2 + vc - 1) / vc) < 512) vc /= 2;
+    dim3 gr((g.nz - 1 + VK - 1) / VK, (g.ny - 1 + VJ - 1) / VJ, (g.gend - 2 + vc - 1) / vc);
+    hipLaunchKernelGGL(k_visc_fused, gr, dim3(VTHREADS), 0, st, U, prof, vF, g, vc, invXI, invET, invZT, inv4XI, inv4ET,
                        inv4ZT);
     return;
   }
