@@ -43,7 +43,7 @@ enum { SET_C = 0, SET_U = 1, SET_V = 2, SET_W = 3 };
 constexpr int PROF_METRIC_ROWS = 40;
 constexpr int FT_REC = PROF_METRIC_ROWS;      // 3 directions x 7 recipes: 1 / sum(w/J)
 constexpr int FT_NRM = FT_REC + 21;           // 3 directions x (insqr, N0, N1, N2) of the face normal
-constexpr int FT_RCP = FT_NRM + 12;          // 3 directions x (rcp_checked of Jf, of insqr)
+constexpr int FT_RCP = FT_NRM + 12;          // 3 directions x (RN(1/Jf), RN(1/insqr))
 constexpr int PROF_ROWS = FT_RCP + 6;
 __device__ __forceinline__ double pf(const double* __restrict__ prof, int Ym, int set, int comp, int j) {
   return prof[(set * 10 + comp) * Ym + j];
@@ -235,39 +235,35 @@ __device__ __forceinline__ void reconstruct(int r, const double (&u)[5][6], cons
 // impermeable-wall face of Flux_Y.cpp:452-460.
 // nt = (insqr, N0, N1, N2) = (1/|n|, n/|n|) of the face, a function of j
 // formed once in the profile rows as 1.0 / sqrt(n.n) and n * insqr
-// FAST: divide by Jf and insqr through their reciprocals rJf, rin
-// (rcp_checked, both non-zero); otherwise plainly
-template <bool FAST>
-__device__ __forceinline__ double div_face(double x, double d, double r) {
-  if (FAST) return div_const(x, d, r);
-  return x / d;
-}
-
-template <bool FAST>
+// rJf, rin: RN(1/Jf), RN(1/insqr).  Quotients with a common divisor share its
+// reciprocal (div_rn, the same bits): a face has 25 divisions, of which 20 have
+// one of five divisors, and a division is about twelve instructions.
 __device__ __forceinline__ void roe_flux(const double L[5], const double Rr[5], const double n[3], const double nt[4],
                                          double Jf, double rJf, double rin, bool energy_norm, bool wall,
                                          double F[5]) {
   const double insqr = nt[0], N0 = nt[1], N1 = nt[2], N2 = nt[3];
-  double _rho = L[0], _u = L[1] / _rho, _v = L[2] / _rho, _w = L[3] / _rho;
+  const double _rho = L[0], _r = 1.0 / _rho;
+  double _u = div_rn(L[1], _rho, _r), _v = div_rn(L[2], _rho, _r), _w = div_rn(L[3], _rho, _r);
   double _U = n[0] * _u + n[1] * _v + n[2] * _w;
   double _VV = _u * _u + _v * _v + _w * _w;
   double _P = (L[4] - 0.5 * _rho * _VV) * (KG - 1);
-  double _C = KG * _P / _rho;
+  double _C = div_rn(KG * _P, _rho, _r);
   double _H = 0.5 * _VV + div_const(_C, KG - 1, RKG);
-  double rho_ = Rr[0], u_ = Rr[1] / rho_, v_ = Rr[2] / rho_, w_ = Rr[3] / rho_;
+  const double rho_ = Rr[0], r_ = 1.0 / rho_;
+  double u_ = div_rn(Rr[1], rho_, r_), v_ = div_rn(Rr[2], rho_, r_), w_ = div_rn(Rr[3], rho_, r_);
   double U_ = n[0] * u_ + n[1] * v_ + n[2] * w_;
   double VV_ = u_ * u_ + v_ * v_ + w_ * w_;
   double P_ = (Rr[4] - 0.5 * rho_ * VV_) * (KG - 1);
-  double C_ = KG * P_ / rho_;
+  double C_ = div_rn(KG * P_, rho_, r_);
   double H_ = 0.5 * VV_ + div_const(C_, KG - 1, RKG);
-  double t5 = sqrt(_rho), t6 = sqrt(rho_), t4 = t5 + t6;
+  const double t5 = sqrt(_rho), t6 = sqrt(rho_), t4 = t5 + t6, rt = 1.0 / t4;
   double rho = sqrt(_rho * rho_);
-  double u = (t5 * _u + t6 * u_) / t4;
-  double v = (t5 * _v + t6 * v_) / t4;
-  double w = (t5 * _w + t6 * w_) / t4;
-  double U = (t5 * _U + t6 * U_) / t4;
+  double u = div_rn(t5 * _u + t6 * u_, t4, rt);
+  double v = div_rn(t5 * _v + t6 * v_, t4, rt);
+  double w = div_rn(t5 * _w + t6 * w_, t4, rt);
+  double U = div_rn(t5 * _U + t6 * U_, t4, rt);
   double VV = u * u + v * v + w * w;
-  double H = (t5 * _H + t6 * H_) / t4;
+  double H = div_rn(t5 * _H + t6 * H_, t4, rt);
   double C = (H - 0.5 * VV) * (KG - 1);
   double dU1 = rho_ - _rho;
   double dU2 = rho_ * u_ - _rho * _u;
@@ -288,16 +284,16 @@ __device__ __forceinline__ void roe_flux(const double L[5], const double Rr[5], 
   if (wall) {
     F[0] = 0;
     F[1] = 0;
-    F[2] = div_face<FAST>(0.5 * (n[1] * (_P + P_) - div_face<FAST>(Fav3, insqr, rin)), Jf, rJf);
+    F[2] = div_rn(0.5 * (n[1] * (_P + P_) - div_rn(Fav3, insqr, rin)), Jf, rJf);
     F[3] = 0;
     F[4] = 0;
     return;
   }
-  F[0] = div_face<FAST>(0.5 * ((_rho * _U + rho_ * U_) - div_face<FAST>(Fav1, insqr, rin)), Jf, rJf);
-  F[1] = div_face<FAST>(0.5 * ((_rho * _u * _U + rho_ * u_ * U_ + n[0] * (_P + P_)) - div_face<FAST>(Fav2, insqr, rin)), Jf, rJf);
-  F[2] = div_face<FAST>(0.5 * ((_rho * _v * _U + rho_ * v_ * U_ + n[1] * (_P + P_)) - div_face<FAST>(Fav3, insqr, rin)), Jf, rJf);
-  F[3] = div_face<FAST>(0.5 * ((_rho * _w * _U + rho_ * w_ * U_ + n[2] * (_P + P_)) - div_face<FAST>(Fav4, insqr, rin)), Jf, rJf);
-  F[4] = div_face<FAST>(0.5 * ((_U * (3.5 * _P + 0.5 * _rho * _VV) + U_ * (3.5 * P_ + 0.5 * rho_ * VV_)) - div_face<FAST>(Fav5, insqr, rin)),
+  F[0] = div_rn(0.5 * ((_rho * _U + rho_ * U_) - div_rn(Fav1, insqr, rin)), Jf, rJf);
+  F[1] = div_rn(0.5 * ((_rho * _u * _U + rho_ * u_ * U_ + n[0] * (_P + P_)) - div_rn(Fav2, insqr, rin)), Jf, rJf);
+  F[2] = div_rn(0.5 * ((_rho * _v * _U + rho_ * v_ * U_ + n[1] * (_P + P_)) - div_rn(Fav3, insqr, rin)), Jf, rJf);
+  F[3] = div_rn(0.5 * ((_rho * _w * _U + rho_ * w_ * U_ + n[2] * (_P + P_)) - div_rn(Fav4, insqr, rin)), Jf, rJf);
+  F[4] = div_rn(0.5 * ((_U * (3.5 * _P + 0.5 * _rho * _VV) + U_ * (3.5 * P_ + 0.5 * rho_ * VV_)) - div_rn(Fav5, insqr, rin)),
                   Jf, rJf);
 }
 
@@ -546,9 +542,10 @@ struct Prim {
 __device__ __forceinline__ Prim prim_visc(double U1, double U2, double U3, double U4, double U5, double J) {
   Prim q;
   double rho = U1;
-  q.U = U2 / rho;
-  q.V = U3 / rho;
-  q.W = U4 / rho;
+  const double r = 1.0 / rho;
+  q.U = div_rn(U2, rho, r);
+  q.V = div_rn(U3, rho, r);
+  q.W = div_rn(U4, rho, r);
   double VV = q.U * q.U + q.V * q.V + q.W * q.W;
   double P = (U5 - 0.5 * rho * VV) * (KG - 1) * J;
   q.T = P / (rho * RG) / J;

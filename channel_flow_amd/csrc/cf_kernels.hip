@@ -91,11 +91,7 @@ __device__ __forceinline__ void flux_face(const double (&u)[5][6], int f, int i,
   double Jf = pf(prof, g.Ym, set, 0, jp);
   bool wall = DIR == 1 && (f == 1 || f == g.ny);
   const double rJf = prow(prof, g.Ym, FT_RCP + 2 * DIR, jp), rin = prow(prof, g.Ym, FT_RCP + 2 * DIR + 1, jp);
-  // a wave covers one face row, so this vote is one branch per wave
-  if (__all(rJf != 0.0 && rin != 0.0))
-    roe_flux<true>(L, R, n, nt, Jf, rJf, rin, DIR == 1, wall, out);
-  else
-    roe_flux<false>(L, R, n, nt, Jf, rJf, rin, DIR == 1, wall, out);
+  roe_flux(L, R, n, nt, Jf, rJf, rin, DIR == 1, wall, out);
 #pragma unroll
   for (int v = 0; v < 5; v++) F[v * g.nf + o] = out[v];
 }
@@ -681,7 +677,7 @@ struct VLds {
   double P[3][4][VR][VKK];
   double ML[4][VJ + 1][VK];
   double NL[4][VJ][VK + 1];
-  double PJ[3][4][VJ + 1];  // face sets U, V, W: xidx, etdy, ztdz and J at j - 1, row j - j0
+  double PJ[3][5][VJ + 1];  // face sets U, V, W: xidx, etdy, ztdz, J and 1 / J at j - 1, row j - j0
 };
 
 __device__ __forceinline__ Prim vp(const VLds& L, int s, int r, int c) {
@@ -761,17 +757,17 @@ __device__ __forceinline__ void vface_x(const VLds& L, int s0, int sm, int r, in
   const double dzu = (lp(L, s0, 0, r, c + 1) + lp(L, sm, 0, r, c + 1) - lp(L, s0, 0, r, c - 1) - lp(L, sm, 0, r, c - 1)) * inv4ZT;
   const double dzw = (lp(L, s0, 2, r, c + 1) + lp(L, sm, 2, r, c + 1) - lp(L, s0, 2, r, c - 1) - lp(L, sm, 2, r, c - 1)) * inv4ZT;
   const DiagCoef m{L.PJ[0][0][r - 1], L.PJ[0][1][r - 1], L.PJ[0][2][r - 1]};
-  const double Jf = L.PJ[0][3][r - 1];
+  const double Jf = L.PJ[0][3][r - 1], rJ = L.PJ[0][4][r - 1];
   const double a1 = (4. / 3) * m.X * m.X, a2 = m.X * m.X, a3 = m.X * m.X, a4 = m.X * m.X;
   const double d5 = m.X * m.E, d7 = -((2. / 3) * m.X * m.E);
   const double e6 = m.X * m.Z, e9 = -((2. / 3) * m.X * m.Z);
   const double Ux = 0.5 * (P0.U + iP.U), Vx = 0.5 * (P0.V + iP.V), Wx = 0.5 * (P0.W + iP.W);
-  o[0] = MU_L * (a1 * dx.u + d7 * dyv + e9 * dzw) / Jf;
-  o[1] = MU_L * (a2 * dx.v + d5 * dyu) / Jf;
-  o[2] = MU_L * (a3 * dx.w + e6 * dzu) / Jf;
-  o[3] = MU_L * (0.5 * a1 * dx.uu + 0.5 * a2 * dx.vv + 0.5 * a3 * dx.ww + CF_CVK_PR(a4, dx.T) + d5 * Vx * dyu +
-                 d7 * Ux * dyv + e6 * Wx * dzu + e9 * Ux * dzw) /
-         Jf;
+  o[0] = div_rn(MU_L * (a1 * dx.u + d7 * dyv + e9 * dzw), Jf, rJ);
+  o[1] = div_rn(MU_L * (a2 * dx.v + d5 * dyu), Jf, rJ);
+  o[2] = div_rn(MU_L * (a3 * dx.w + e6 * dzu), Jf, rJ);
+  o[3] = div_rn(MU_L * (0.5 * a1 * dx.uu + 0.5 * a2 * dx.vv + 0.5 * a3 * dx.ww + CF_CVK_PR(a4, dx.T) + d5 * Vx * dyu +
+                 d7 * Ux * dyv + e6 * Wx * dzu + e9 * Ux * dzw),
+                Jf, rJ);
 }
 
 // y face between rows r-1 and r of plane slot s0
@@ -784,17 +780,17 @@ __device__ __forceinline__ void vface_y(const VLds& L, int sp, int s0, int sm, i
   const double dzv = (lp(L, s0, 1, r, c + 1) + lp(L, s0, 1, r - 1, c + 1) - lp(L, s0, 1, r, c - 1) - lp(L, s0, 1, r - 1, c - 1)) * inv4ZT;
   const double dzw = (lp(L, s0, 2, r, c + 1) + lp(L, s0, 2, r - 1, c + 1) - lp(L, s0, 2, r, c - 1) - lp(L, s0, 2, r - 1, c - 1)) * inv4ZT;
   const DiagCoef m{L.PJ[1][0][r - 1], L.PJ[1][1][r - 1], L.PJ[1][2][r - 1]};
-  const double Jf = L.PJ[1][3][r - 1];
+  const double Jf = L.PJ[1][3][r - 1], rJ = L.PJ[1][4][r - 1];
   const double b1 = m.E * m.E, b2 = (4. / 3) * m.E * m.E, b3 = m.E * m.E, b4 = m.E * m.E;
   const double d5 = m.X * m.E, d7 = -((2. / 3) * m.X * m.E);
   const double f8 = m.E * m.Z, f10 = -((2. / 3) * m.E * m.Z);
   const double Uy = 0.5 * (P0.U + jP.U), Vy = 0.5 * (P0.V + jP.V), Wy = 0.5 * (P0.W + jP.W);
-  o[0] = MU_L * (d5 * dxv + b1 * dy.u) / Jf;
-  o[1] = MU_L * (d7 * dxu + b2 * dy.v + f10 * dzw) / Jf;
-  o[2] = MU_L * (b3 * dy.w + f8 * dzv) / Jf;
-  o[3] = MU_L * (0.5 * b1 * dy.uu + 0.5 * b2 * dy.vv + 0.5 * b3 * dy.ww + CF_CVK_PR(b4, dy.T) + d5 * Uy * dxv +
-                 d7 * Vy * dxu + f8 * Wy * dzv + f10 * Vy * dzw) /
-         Jf;
+  o[0] = div_rn(MU_L * (d5 * dxv + b1 * dy.u), Jf, rJ);
+  o[1] = div_rn(MU_L * (d7 * dxu + b2 * dy.v + f10 * dzw), Jf, rJ);
+  o[2] = div_rn(MU_L * (b3 * dy.w + f8 * dzv), Jf, rJ);
+  o[3] = div_rn(MU_L * (0.5 * b1 * dy.uu + 0.5 * b2 * dy.vv + 0.5 * b3 * dy.ww + CF_CVK_PR(b4, dy.T) + d5 * Uy * dxv +
+                 d7 * Vy * dxu + f8 * Wy * dzv + f10 * Vy * dzw),
+                Jf, rJ);
 }
 
 // z face between columns c-1 and c of plane slot s0
@@ -807,17 +803,17 @@ __device__ __forceinline__ void vface_z(const VLds& L, int sp, int s0, int sm, i
   const double dyv = (lp(L, s0, 1, r + 1, c) + lp(L, s0, 1, r + 1, c - 1) - lp(L, s0, 1, r - 1, c) - lp(L, s0, 1, r - 1, c - 1)) * inv4ET;
   const double dyw = (lp(L, s0, 2, r + 1, c) + lp(L, s0, 2, r + 1, c - 1) - lp(L, s0, 2, r - 1, c) - lp(L, s0, 2, r - 1, c - 1)) * inv4ET;
   const DiagCoef m{L.PJ[2][0][r - 1], L.PJ[2][1][r - 1], L.PJ[2][2][r - 1]};
-  const double Jf = L.PJ[2][3][r - 1];
+  const double Jf = L.PJ[2][3][r - 1], rJ = L.PJ[2][4][r - 1];
   const double c1 = m.Z * m.Z, c2 = m.Z * m.Z, c3 = (4. / 3) * m.Z * m.Z, c4 = m.Z * m.Z;
   const double e6 = m.X * m.Z, e9 = -((2. / 3) * m.X * m.Z);
   const double f8 = m.E * m.Z, f10 = -((2. / 3) * m.E * m.Z);
   const double Uz = 0.5 * (P0.U + kP.U), Vz = 0.5 * (P0.V + kP.V), Wz = 0.5 * (P0.W + kP.W);
-  o[0] = MU_L * (e6 * dxw + c1 * dz.u) / Jf;
-  o[1] = MU_L * (f8 * dyw + c2 * dz.v) / Jf;
-  o[2] = MU_L * (e9 * dxu + f10 * dyv + c3 * dz.w) / Jf;
-  o[3] = MU_L * (0.5 * c1 * dz.uu + 0.5 * c2 * dz.vv + 0.5 * c3 * dz.ww + CF_CVK_PR(c4, dz.T) + e6 * Uz * dxw +
-                 e9 * Wz * dxu + f8 * Vz * dyw + f10 * Wz * dyv) /
-         Jf;
+  o[0] = div_rn(MU_L * (e6 * dxw + c1 * dz.u), Jf, rJ);
+  o[1] = div_rn(MU_L * (f8 * dyw + c2 * dz.v), Jf, rJ);
+  o[2] = div_rn(MU_L * (e9 * dxu + f10 * dyv + c3 * dz.w), Jf, rJ);
+  o[3] = div_rn(MU_L * (0.5 * c1 * dz.uu + 0.5 * c2 * dz.vv + 0.5 * c3 * dz.ww + CF_CVK_PR(c4, dz.T) + e6 * Uz * dxw +
+                 e9 * Wz * dxu + f8 * Vz * dyw + f10 * Wz * dyv),
+                Jf, rJ);
 }
 
 __global__ void __launch_bounds__(VTHREADS) k_visc_fused(const double* __restrict__ U,
@@ -851,7 +847,9 @@ __global__ void __launch_bounds__(VTHREADS) k_visc_fused(const double* __restric
     L.PJ[set][0][r] = in ? pf(prof, g.Ym, sid, 1, jp) : 0.;
     L.PJ[set][1][r] = in ? pf(prof, g.Ym, sid, 5, jp) : 0.;
     L.PJ[set][2][r] = in ? pf(prof, g.Ym, sid, 9, jp) : 0.;
-    L.PJ[set][3][r] = in ? pf(prof, g.Ym, sid, 0, jp) : 0.;
+    const double Jf = in ? pf(prof, g.Ym, sid, 0, jp) : 0.;
+    L.PJ[set][3][r] = Jf;
+    L.PJ[set][4][r] = 1.0 / Jf;
   }
   VRaw R;
   vfetch(R, U, prof, g, ib - 1, j0, k0, tid);
@@ -2568,7 +2566,7 @@ void launch_halo_bc(hipStream_t st, double* U, const double* prof, const Geo& g,
 // the cell's j along x and z, at face j along y; stencil J clamped to the
 // array for recipes a face does not use), FT_NRM + 4 d the face normal's
 // (insqr, N0, N1, N2) at the face row the fluxes read, FT_RCP + 2 d the
-// checked reciprocals of that row's face J and insqr
+// reciprocals of that row's face J and insqr
 __global__ void k_flux_tables(double* __restrict__ prof, Geo g) {
   const int idx = blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= 24 * g.Ym) return;
@@ -2588,8 +2586,8 @@ __global__ void k_flux_tables(double* __restrict__ prof, Geo g) {
     prof[(long)(FT_NRM + 4 * d + 1) * g.Ym + j] = n0 * insqr;
     prof[(long)(FT_NRM + 4 * d + 2) * g.Ym + j] = n1 * insqr;
     prof[(long)(FT_NRM + 4 * d + 3) * g.Ym + j] = n2 * insqr;
-    prof[(long)(FT_RCP + 2 * d) * g.Ym + j] = rcp_checked(pf(prof, g.Ym, set, 0, j));
-    prof[(long)(FT_RCP + 2 * d + 1) * g.Ym + j] = rcp_checked(insqr);
+    prof[(long)(FT_RCP + 2 * d) * g.Ym + j] = 1.0 / pf(prof, g.Ym, set, 0, j);
+    prof[(long)(FT_RCP + 2 * d + 1) * g.Ym + j] = 1.0 / insqr;
   }
 }
 
