@@ -141,8 +141,9 @@ struct cf_ctx {
   // the NL slots that the single-wave tiles hand across hold the sentinel
   bool tiles_seeded = false;
   double* partial = nullptr;
-  double* er_dev = nullptr;   // the norms, then the two sweep error flags
-  double* er_host = nullptr;  // pinned copy of er_dev, read after each iteration
+  // the norms, then the two sweep error flags, in pinned memory that the last
+  // reduction writes: the host's and the device's address
+  double *er_host = nullptr, *er_dev = nullptr;
   double* pin = nullptr;      // pinned buffer for small host arrays (PIN_ELEMS)
   double* stat = nullptr;  // running per-j sums of Statistic's mean profiles (7 * Ym)
   double* shear = nullptr; // wall values of Statistic's y-face viscous flux (2 * X_out * Z_out)
@@ -398,8 +399,9 @@ extern "C" int cf_create(const cf_params* p, cf_ctx** out) {
   }
   long nb = std::max(cf::update_blocks(g), cf::sweep_update_blocks(g));
   if (hipMalloc(&c->partial, (size_t)nb * 5 * sizeof(double)) != hipSuccess) return bail(CF_ERR_HIP);
-  if (hipMalloc(&c->er_dev, 8 * sizeof(double)) != hipSuccess) return bail(CF_ERR_HIP);
-  if (hipHostMalloc(&c->er_host, 8 * sizeof(double), hipHostMallocDefault) != hipSuccess) return bail(CF_ERR_HIP);
+  if (hipHostMalloc(&c->er_host, 8 * sizeof(double), hipHostMallocMapped) != hipSuccess ||
+      hipHostGetDevicePointer((void**)&c->er_dev, c->er_host, 0) != hipSuccess)
+    return bail(CF_ERR_HIP);
   if (hipHostMalloc(&c->pin, PIN_ELEMS * sizeof(double), hipHostMallocDefault) != hipSuccess) return bail(CF_ERR_HIP);
   if (hipMalloc(&c->stat, (size_t)7 * g.Ym * sizeof(double)) != hipSuccess) return bail(CF_ERR_HIP);
   if (hipMalloc(&c->shear, (size_t)2 * p->X_out * p->Z_out * sizeof(double)) != hipSuccess) return bail(CF_ERR_HIP);
@@ -425,7 +427,7 @@ extern "C" void cf_destroy(cf_ctx* c) {
   }
   if (c->fork_ev) (void)hipEventDestroy(c->fork_ev);
   double* ptrs[] = {c->Ui, c->Un, c->Uq, c->Fx, c->Fy, c->Fz, c->vF, c->MR,  c->NL,     c->NR,    c->Pr,
-                    c->VS, c->Ep, c->Fw, c->ypt, c->Sm, c->partial, c->er_dev, c->prof, c->stat, c->Uqq, c->Hs, c->U3, c->Ualt, c->shear};
+                    c->VS, c->Ep, c->Fw, c->ypt, c->Sm, c->partial, c->prof, c->stat, c->Uqq, c->Hs, c->U3, c->Ualt, c->shear};
   for (double* q : ptrs)
     if (q) (void)hipFree(q);
   if (c->order) (void)hipFree(c->order);
@@ -900,10 +902,8 @@ static void update(cf_ctx* c) {
 }
 
 // er to the host and the sweep error flags checked
-// (one copy into pinned memory: the norms and the flags, which the last
-// reduction kernel placed after them)
+// (the last reduction kernel writes both to pinned memory)
 static int finish_iteration(cf_ctx* c, double er[5]) {
-  HIPCHK(c, hipMemcpyAsync(c->er_host, c->er_dev, 7 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   int r = sync(c);
   if (r) {
     c->hand_off = 0;
@@ -931,7 +931,6 @@ static int dplusgs_device(cf_ctx* c, double deltaT, double er[5]) {
   cf::launch_dplusgs(c->stream, c->Ui, c->MR, c->NL, c->NR, c->prof, g, deltaT);
   double DN = 1. / ((double)c->p.X_out * c->p.Y_out * c->p.Z_out);
   cf::launch_update(c->stream, c->Ui, c->NR, c->prof, c->partial, c->er_dev, g, DN);
-  HIPCHK(c, hipMemcpyAsync(c->er_host, c->er_dev, 5 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   int r = sync(c);
   if (r) return r;
   for (int v = 0; v < 5; v++) er[v] = c->er_host[v];
@@ -1125,6 +1124,16 @@ extern "C" int cf_read_state(cf_ctx* c, double* const Qn[5], double* const Qnm1[
   return CF_OK;
 }
 
+// Whether the stencils run on four streams.  The fork and join cost seven event
+// calls eagerly (about 30 us: 16x12x16 124 us an iteration on one stream, 155
+// on four; 64^3 337 and 357; 128x96x128 855 and 871; 256x192x256 4301 and
+// 4277) and little in a graph (48^3 256 and 263; 56^3 298 and 292; 256x192x256
+// 4311 and 4246).
+static bool fork_pays(const cf_ctx* c) {
+  const long cells = (long)c->p.X_out * c->p.Y_out * c->p.Z_out;
+  return cells >= (c->use_graph ? 150000 : 4000000);
+}
+
 // Everything one inner iteration of the device state launches: kernels
 // only, no copies, no memsets and no synchronisation, so that the sequence
 // can be captured into a graph.  The checks and allocations it could need
@@ -1132,7 +1141,7 @@ extern "C" int cf_read_state(cf_ctx* c, double* const Qn[5], double* const Qnm1[
 static int prepare_iteration(cf_ctx* c) {
   if (!viscous_fused(c))
     if (int r = ensure_viscous_staging(c)) return r;
-  if (c->fork && !c->fork_ev) {
+  if (c->fork && fork_pays(c) && !c->fork_ev) {
     for (int q = 0; q < 3; q++) {
       HIPCHK(c, hipStreamCreateWithFlags(&c->aux[q], hipStreamNonBlocking));
       HIPCHK(c, hipEventCreateWithFlags(&c->join_ev[q], hipEventDisableTiming));
@@ -1148,7 +1157,7 @@ static int prepare_iteration(cf_ctx* c) {
 static void enqueue_iteration(cf_ctx* c) {
   const Geo& g = c->g;
   cf::launch_halo_bc(c->stream, c->Ui, c->prof, g, c->p.x_periodic);
-  if (c->fork && c->fork_ev) {
+  if (c->fork && c->fork_ev && fork_pays(c)) {
     // Flux_X on the context's stream, Flux_Y, Flux_Z and Viscous_terms on
     // the helper streams, all after the ghost cells, all before the RHS
     (void)hipEventRecord(c->fork_ev, c->stream);
@@ -1353,7 +1362,7 @@ extern "C" int cf_profile_inner_iteration(cf_ctx* c, double er[5], double stage_
   if ((r = span(mk[nm - 1], ev[7 + nm], &stage_ms[10]))) return r;
   const bool tiled = effective_schedule(c) == 0;
   const int nplanes = g.gend + g.ny + g.nz - 6;
-  const int nl[CF_PROFILE_STAGES] = {3, 1, 1, 1, viscous_fused(c) ? 1 : 3, fuse ? 0 : 1, tiled ? 1 : 0, tiled ? ns : 0, tiled ? ns : nplanes * ns,
+  const int nl[CF_PROFILE_STAGES] = {1, 1, 1, 1, viscous_fused(c) ? 1 : 3, fuse ? 0 : 1, tiled ? 1 : 0, tiled ? ns - 1 : 0, tiled ? ns : nplanes * ns,
                                      tiled ? ns : nplanes * ns, 2};
   for (int q = 0; q < CF_PROFILE_STAGES; q++) launches[q] = nl[q];
   return CF_OK;

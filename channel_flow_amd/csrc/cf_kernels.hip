@@ -18,47 +18,75 @@ namespace cf {
 // ghost cells: main.cpp:203-240 (x), Y_boundary_condition.cpp:48-120 (walls),
 // Z_boundary_condition.cpp:48-66 (periodic z)
 // ---------------------------------------------------------------------------
-__global__ void k_halo_x(double* __restrict__ U, Geo g, int src_lo, int src_hi) {
-  long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= g.plane) return;
-  double* f = U + (long)blockIdx.y * g.nf;
-  if (blockIdx.z == 0)
-    f[2 * g.plane + idx] = f[(long)src_lo * g.plane + idx];
-  else
-    f[(long)(g.gend + 1) * g.plane + idx] = f[(long)src_hi * g.plane + idx];
-}
-
-__global__ void k_wall(double* __restrict__ U, const double* __restrict__ prof, Geo g) {
-  int k = 2 + blockIdx.x * blockDim.x + threadIdx.x;
-  int i = 2 + blockIdx.y;
-  int s = blockIdx.z;  // 0: bottom (ghost 1 from 2), 1: top (ghost nyy from ny)
-  if (k > g.nz || i > g.gend + 1) return;
-  int ja = s == 0 ? 2 : g.ny, jb = s == 0 ? 1 : g.ny + 1;
-  long a = at(g, i, ja, k), b = at(g, i, jb, k);
-  double Ja = pf(prof, g.Ym, SET_C, 0, ja), Jb = pf(prof, g.Ym, SET_C, 0, jb);
-  double U1 = U[a], U2 = U[g.nf + a], U3 = U[2 * g.nf + a], U4 = U[3 * g.nf + a], U5 = U[4 * g.nf + a];
+// The wall ghost of the cell (is, ja, k): rho, velocities and energy of the
+// mirrored state at the wall temperature, over Jb
+__device__ __forceinline__ void wall_ghost(const double* __restrict__ U, const double* __restrict__ prof, const Geo& g,
+                                           int is, int top, int k, double o[5]) {
+  const int ja = top ? g.ny : 2, jb = top ? g.ny + 1 : 1;
+  const long a = at(g, is, ja, k);
+  const double Ja = pf(prof, g.Ym, SET_C, 0, ja), Jb = pf(prof, g.Ym, SET_C, 0, jb);
+  const double U1 = U[a], U2 = U[g.nf + a], U3 = U[2 * g.nf + a], U4 = U[3 * g.nf + a], U5 = U[4 * g.nf + a];
   double rho = U1 * Ja;
-  double Uu = U2 / U1, V = U3 / U1, W = U4 / U1;
-  double VV = Uu * Uu + V * V + W * W;
-  double P = (U5 * Ja - 0.5 * rho * VV) * (KG - 1);
-  double temp = P / rho / RG;
-  double T = T_WALL2 - temp;
+  const double Uu = U2 / U1, V = U3 / U1, W = U4 / U1;
+  const double VV = Uu * Uu + V * V + W * W;
+  const double P = (U5 * Ja - 0.5 * rho * VV) * (KG - 1);
+  const double temp = P / rho / RG;
+  const double T = T_WALL2 - temp;
   rho = P / RG / T;
-  U[b] = P / RG / T / Jb;
-  U[g.nf + b] = -P / RG / T * Uu / Jb;
-  U[2 * g.nf + b] = -P / RG / T * V / Jb;
-  U[3 * g.nf + b] = -P / RG / T * W / Jb;
-  U[4 * g.nf + b] = (rho * RG * T / (KG - 1) + 0.5 * P / RG / T * VV) / Jb;
+  o[0] = P / RG / T / Jb;
+  o[1] = -P / RG / T * Uu / Jb;
+  o[2] = -P / RG / T * V / Jb;
+  o[3] = -P / RG / T * W / Jb;
+  o[4] = (rho * RG * T / (KG - 1) + 0.5 * P / RG / T * VV) / Jb;
 }
 
-__global__ void k_zper(double* __restrict__ U, Geo g) {
-  int j = blockIdx.x * blockDim.x + threadIdx.x;  // 0 .. nyyy
-  int i = 2 + blockIdx.y;
-  int v = blockIdx.z;
-  if (j > g.ny + 2 || i > g.gend + 1) return;
-  double* f = U + (long)v * g.nf;
-  f[at(g, i, j, 1)] = f[at(g, i, j, g.nz)];
-  f[at(g, i, j, g.nz + 1)] = f[at(g, i, j, 2)];
+// All ghost cells in one launch.  The reference copies the x ghost planes,
+// then forms the walls' ghosts (the x ghost planes' too), then copies the
+// periodic z ghosts (the walls' too); every one of them follows from cells
+// that stay as they are: plane is = src_lo, src_hi or i, column k' = nz, 2 or
+// k, and at j = 1, ny + 1 the wall's mirror of (is, ., k').  Threads: the two
+// x ghost planes, then the wall rows, then the z columns of the others.
+// In place of three launches: 35 -> 29 us at 256x192x256, 12 -> 8 us at
+// 16x12x16.
+__global__ void __launch_bounds__(256) k_ghosts(double* __restrict__ U, const double* __restrict__ prof, Geo g,
+                                                int src_lo, int src_hi) {
+  const int Z = g.nz - 1, X = g.gend - 2;
+  const long nx = 2 * g.plane, nw = (long)X * 2 * Z, nc = (long)X * (g.ny + 3) * 2;
+  long t = (long)blockIdx.x * 256 + threadIdx.x;
+  int i, j, k, is;
+  if (t < nx) {
+    const int hi = t >= g.plane;
+    const long e = t - (hi ? g.plane : 0);
+    i = hi ? g.gend + 1 : 2;
+    is = hi ? src_hi : src_lo;
+    j = (int)(e / g.Zp);
+    k = (int)(e - (long)j * g.Zp);
+  } else if ((t -= nx) < nw) {
+    const long r = t / Z;
+    k = 2 + (int)(t - r * Z);
+    j = r & 1 ? g.ny + 1 : 1;
+    i = is = 3 + (int)(r >> 1);
+  } else if ((t -= nw) < nc) {
+    const long r = t >> 1;
+    k = t & 1 ? g.nz + 1 : 1;
+    i = (int)(r / (g.ny + 3));
+    j = (int)(r - (long)i * (g.ny + 3));
+    i = is = 3 + i;
+  } else {
+    return;
+  }
+  const int ks = k == 1 ? g.nz : k == g.nz + 1 ? 2 : k;
+  double o[5];
+  if ((j == 1 || j == g.ny + 1) && ks >= 2 && ks <= g.nz) {
+    wall_ghost(U, prof, g, is, j != 1, ks, o);
+  } else {
+    const long a = at(g, is, j, ks);
+#pragma unroll
+    for (int v = 0; v < 5; v++) o[v] = U[v * g.nf + a];
+  }
+  const long b = at(g, i, j, k);
+#pragma unroll
+  for (int v = 0; v < 5; v++) U[v * g.nf + b] = o[v];
 }
 
 // ---------------------------------------------------------------------------
@@ -1206,6 +1234,16 @@ __device__ __forceinline__ void store_summary(T* __restrict__ S, T* __restrict__
   }
 }
 
+// tickets, error flags and progress of both sweep directions back to zero: by
+// the pre-pass's first block for the first sweep pair, by k_sweep_reset before
+// each later one
+__device__ __forceinline__ void sweep_reset(int* __restrict__ sync, int n) {
+  if (blockIdx.x == 0 && blockIdx.y == 0)
+    for (int t = threadIdx.x; t < n; t += blockDim.x) sync[t] = 0;
+}
+
+__global__ void __launch_bounds__(256) k_sweep_reset(int* __restrict__ sync, int n) { sweep_reset(sync, n); }
+
 // A prep block covers PC steps of one tile.  Column (a, b) of the tile meets
 // cells k-2 = s - a - b at steps s0 .. s0+PC-1: one run of PC consecutive k,
 // which the block stages in LDS with coalesced loads; slot (s, lane) then
@@ -1234,8 +1272,10 @@ __device__ __forceinline__ void prep_stage(double (*L)[64][PCP], const double* _
 template <class T>
 __global__ void __launch_bounds__(256) k_sweep_prep(const double* __restrict__ Ui, const double* __restrict__ MR,
                                                     const double* __restrict__ prof, T* __restrict__ S,
-                                                    T* __restrict__ MRs, T* __restrict__ E, Geo g, Sk q) {
+                                                    T* __restrict__ MRs, T* __restrict__ E, Geo g, Sk q,
+                                                    int* __restrict__ sync) {
   __shared__ double L[5][64][PCP];
+  sweep_reset(sync, 2 * q.ntiles + 4);
   int bx, by, bz;
   xcd_block3(&bx, &by, &bz);
   const int tile = by, s0 = bx * PC;
@@ -1283,7 +1323,8 @@ template <class T>
 __global__ void __launch_bounds__(PR_THREADS) k_sweep_prep_rhs(const double* __restrict__ Ui, RhsIn rin,
                                                                const double* __restrict__ prof, T* __restrict__ S,
                                                                T* __restrict__ MRs, T* __restrict__ E, Geo g, Sk q,
-                                                               double deltaT) {
+                                                               double deltaT, int* __restrict__ sync) {
+  sweep_reset(sync, 2 * q.ntiles + 4);
   __shared__ double L[5][64][PRP];
   int bx, by, bz;
   xcd_block3(&bx, &by, &bz);
@@ -1363,11 +1404,6 @@ __global__ void __launch_bounds__(256) k_seed_tiles(double* __restrict__ NLs, Sk
   const double sv = sentinel_value<double>();
 #pragma unroll
   for (int v = 0; v < 5; v++) NLs[v * q.nsk + o] = sv;
-}
-
-__global__ void k_sweep_reset(int* __restrict__ sync, int n) {
-  int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) sync[t] = 0;
 }
 
 __device__ __forceinline__ double ld_coherent(const double* p) {
@@ -2556,9 +2592,8 @@ void launch_q_out(hipStream_t st, const double* U, const double* J, double* Q, c
 
 void launch_halo_bc(hipStream_t st, double* U, const double* prof, const Geo& g, int x_periodic) {
   int src_lo = x_periodic ? g.gend : 3, src_hi = x_periodic ? 3 : g.gend;
-  hipLaunchKernelGGL(k_halo_x, dim3((unsigned)((g.plane + 255) / 256), 5, 2), dim3(256), 0, st, U, g, src_lo, src_hi);
-  hipLaunchKernelGGL(k_wall, dim3((g.nz - 1 + 63) / 64, g.gend, 2), dim3(64), 0, st, U, prof, g);
-  hipLaunchKernelGGL(k_zper, dim3((g.ny + 3 + 63) / 64, g.gend, 5), dim3(64), 0, st, U, g);
+  const long n = 2 * g.plane + (long)(g.gend - 2) * (2 * (g.nz - 1) + 2 * (g.ny + 3));
+  hipLaunchKernelGGL(k_ghosts, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, U, prof, g, src_lo, src_hi);
 }
 
 // derived profile rows for the fluxes, recomputed whenever the metric rows
@@ -2947,14 +2982,14 @@ static void sweeps_t(hipStream_t st, double* Ui, const double* MR, double* Sbuf,
   T* E = H + ho_at(q, q.ntiles, 0, 0);
   if (rin)
     hipLaunchKernelGGL(k_sweep_prep_rhs<T>, dim3((q.nsteps + PR - 1) / PR, q.ntiles), dim3(PR_THREADS), 0, st, Ui, *rin,
-                       prof, S, MRs, E, g, q, deltaT);
+                       prof, S, MRs, E, g, q, deltaT, sync);
   else
     hipLaunchKernelGGL(k_sweep_prep<T>, dim3((q.nsteps + PC - 1) / PC, q.ntiles), dim3(256), 0, st, Ui, MR, prof, S,
-                       MRs, E, g, q);
+                       MRs, E, g, q, sync);
   if (marks) (void)hipEventRecord(marks[0], st);
   const int nt = q.ntiles;
   for (int sweep = 0; sweep < n_sweeps; sweep++) {
-    hipLaunchKernelGGL(k_sweep_reset, dim3((2 * nt + 4 + 255) / 256), dim3(256), 0, st, sync, 2 * nt + 4);
+    if (sweep > 0) hipLaunchKernelGGL(k_sweep_reset, dim3(1), dim3(256), 0, st, sync, 2 * nt + 4);
     if (marks) (void)hipEventRecord(marks[1 + 3 * sweep], st);
     if constexpr (std::is_same<T, double>::value) {
       if (!pipelined)

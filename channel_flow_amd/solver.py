@@ -469,7 +469,8 @@ class Solver:
         self._chk(self.lib.cf_set_graph(self._h, int(bool(enabled))))
 
     def set_concurrent_stencils(self, enabled: bool = True):
-        """Fluxes and viscous terms on four streams (same bits)."""
+        """Fluxes and viscous terms on four streams where the grid is large
+        enough for that to pay (same bits)."""
         self._chk(self.lib.cf_set_concurrent_stencils(self._h, int(bool(enabled))))
 
     def graph_builds(self) -> int:

@@ -238,7 +238,8 @@ int cf_profile_variants(cf_ctx* ctx, double Roe_criterion, double ms[CF_VARIANT_
 /* Visiting order of the LU-SGS sweeps; all give identical bits because each
  * cell depends only on its three upstream neighbours.  schedule 0 (default):
  * one persistent launch per sweep direction, 8x8-column tiles walking k in
- * dependency order, each tile one compute wave fed by three loader waves;
+ * dependency order, each tile ten wavefronts: loads, polls, computation and
+ * stores on their own;
  * schedule 1: one launch per hyperplane i+j+k = m (the reference order,
  * Hyperplane.cpp:50-78); schedule 2: the tiles of schedule 0 as single waves
  * that load their own inputs.  A CF_FP32_SWEEPS context accepts schedule 0
@@ -333,7 +334,8 @@ int cf_graph_builds(cf_ctx* ctx, long long* builds);
  * Flux_Z and Viscous_terms, which all read the state after its ghost cells
  * and write disjoint outputs, concurrently on the context's stream and three
  * helper streams of default priority (fork and join by events, also inside
- * the graph); 0 runs them one after another.  Same bits either way. */
+ * the graph) where the grid is large enough for that to pay (4 million cells,
+ * in a graph 150000); 0 runs them one after another.  Same bits either way. */
 int cf_set_concurrent_stencils(cf_ctx* ctx, int enabled);
 
 /* --- learned initial iterate ------------------------------------------------
