@@ -188,7 +188,7 @@ static int sync(cf_ctx* c) {
 // summary and MR part, which holds nothing between sweeps.  Every use is
 // ordered on the context's stream.
 static int stage_fields(const cf_ctx* c, long elems) {
-  return (int)std::min(16L, std::max(1L, cf::sweep_scratch_elems(c->g) / elems));
+  return (int)std::min(16L, std::max(1L, cf::sweep_scratch_elems(c->g, c->fp32) / elems));
 }
 
 // n host fields of `elems` doubles each -> the staging copy, in the stream's

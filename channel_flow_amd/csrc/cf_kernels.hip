@@ -2954,8 +2954,9 @@ int sweep_tiles(const Geo& g, int* nTI, int* nTJ) {
 
 long sweep_field_elems(const Geo& g) { return sweep_layout(g).nsk; }
 
-// (S + MR: rewritten by every sweep's pre-pass and read by no one after it)
-long sweep_scratch_elems(const Geo& g) { return (G_N + 5) * sweep_layout(g).nsk; }
+// (S + MR: rewritten by every sweep's pre-pass and read by no one after it; a
+// float layout has half the bytes, and what follows it is kept)
+long sweep_scratch_elems(const Geo& g, bool fp32) { return (G_N + 5) * sweep_layout(g).nsk / (fp32 ? 2 : 1); }
 
 long sweep_buffer_elems(const Geo& g) {
   const Sk q = sweep_layout(g);

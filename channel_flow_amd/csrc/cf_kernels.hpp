@@ -48,7 +48,7 @@ void launch_rhs(hipStream_t st, const double* Ui, const double* Un, const double
 int sweep_tiles(const Geo& g, int* nTI, int* nTJ);
 long sweep_field_elems(const Geo& g);
 long sweep_buffer_elems(const Geo& g);   // doubles in Sbuf
-long sweep_scratch_elems(const Geo& g);  // doubles at its start that hold nothing between sweeps
+long sweep_scratch_elems(const Geo& g, bool fp32);  // doubles at its start that hold nothing between sweeps
 long sweep_update_blocks(const Geo& g);
 // inputs of the RHS, for the sweep pre-pass that forms MR itself (rin)
 struct RhsIn {

@@ -34,3 +34,29 @@ def test_gpu_schedule_switches_keep_the_bits(grid):
                 s.inner_iteration()
             states.append(s.read_state()[2])
     np.testing.assert_array_equal(states[0], states[1])
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_gpu_host_arrays_between_iterations_leave_the_sweeps_alone(precision):
+    """The staging of host arrays shares memory with the sweeps' fields, which
+    take half of it in FP32: arrays that pass through it between two
+    iterations change nothing."""
+    from channel_flow_amd.config import ChannelConfig, FlowParams, poiseuille_state
+    from channel_flow_amd.solver import Solver
+    print(f"host arrays between iterations, precision {precision}", flush=True)
+    cfg = ChannelConfig(40, 36, 24, gamma_metric=2.0, deltaT=1e-8)
+    Q = poiseuille_state(cfg, FlowParams(), seed=11, stream=0)
+    got = []
+    for between in (False, True):
+        with Solver(cfg, precision=precision) as s:
+            s.Jacobian_all(2.0, want_arrays=False)
+            s.load_state(Q, Q)
+            er = []
+            for _ in range(3):
+                er.append(s.inner_iteration())
+                if between:
+                    s.Jacobian_all(2.0)
+                    s.read_state()
+            got.append((np.array(er), s.read_state()[2]))
+    np.testing.assert_array_equal(got[0][0], got[1][0])
+    np.testing.assert_array_equal(got[0][1], got[1][1])
