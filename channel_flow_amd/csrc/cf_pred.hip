@@ -62,7 +62,8 @@ extern "C" int cf_pred_create(int dataset_crops, int batch_crops, cf_pred** out)
       dalloc(&p->x, (size_t)p->B * n3 * cfp::CIN) || dalloc(&p->h1, (size_t)p->B * n3 * cfp::CH) ||
       dalloc(&p->dz2, (size_t)p->B * n3 * cfp::CH) || dalloc(&p->z2, (size_t)p->B * ni3 * cfp::CH) ||
       dalloc(&p->tgt, (size_t)p->B * ni3 * cfp::COUT) || dalloc(&p->part_h, (size_t)hb * cfp::HEAD_PART) ||
-      dalloc(&p->part_d, (size_t)db * cfp::NW1) || dalloc(&p->part_w, (size_t)p->splits * cfp::NW2))
+      dalloc(&p->along_k, (size_t)cfp::along_k_elems(v)) || dalloc(&p->part_d, (size_t)db * cfp::NW1) ||
+      dalloc(&p->part_w, (size_t)p->splits * cfp::NW2))
     return bail(CF_ERR_HIP);
   // dz2 is written on the inner cells only: its margin stays zero
   if (hipMemsetAsync(p->dz2, 0, (size_t)p->B * n3 * cfp::CH * 2, p->stream) != hipSuccess ||
@@ -82,7 +83,7 @@ extern "C" void cf_pred_destroy(cf_pred* p) {
   if (!p) return;
   if (p->stream) (void)hipStreamSynchronize(p->stream);
   void* ptrs[] = {p->P,  p->G,   p->M,   p->V,   p->W1b,    p->W2b,    p->W2Tb,   p->D,     p->x,
-                  p->h1, p->dz2, p->z2, p->tgt, p->part_h, p->part_d, p->part_w, p->losses};
+                  p->h1, p->dz2, p->along_k, p->z2, p->tgt, p->part_h, p->part_d, p->part_w, p->losses};
   for (void* q : ptrs)
     if (q) (void)hipFree(q);
   if (p->stream) (void)hipStreamDestroy(p->stream);
@@ -205,14 +206,14 @@ extern "C" int cf_pred_fit_norm(cf_pred* p, int n, double stats[CF_PRED_NSTATS])
 // pointwise layer, the forward conv, the loss head, both backward convs and
 // the ordered reduction into G (summed squared error at G[NPARAM])
 static void batch_gradient(cf_pred* p, int n, unsigned short* x, unsigned short* h1, float* z2, float* tgt,
-                           unsigned short* dz2, float* ph, float* pd, float* pw) {
+                           unsigned short* dz2, unsigned short* ak, float* ph, float* pd, float* pw) {
   const cfp::Vol v = pred_batch_vol(n, p->VC);
   const float inv_norm = 2.0f / (5.0f * (float)v.inner_cells());
   cfp::launch_l1(p->stream, v, x, p->W1b, h1);
   cfp::launch_fwd(p->stream, v, h1, false, p->W1b, p->W2b, p->P, z2, true);
   const int hb = cfp::launch_head(p->stream, v, z2, tgt, p->P, inv_norm, dz2, ph);
   const int db = cfp::launch_bwd_data(p->stream, v, dz2, p->W2Tb, x, pd);
-  cfp::launch_bwd_weight(p->stream, v, dz2, h1, p->splits, pw);
+  cfp::launch_bwd_weight(p->stream, v, dz2, h1, p->splits, ak, pw);
   cfp::launch_reduce(p->stream, ph, hb, pd, db, pw, p->splits, p->G);
 }
 
@@ -227,7 +228,7 @@ extern "C" int cf_pred_train(cf_pred* p, int n_train, int steps, float lr, unsig
   }
   for (int s = 0; s < steps; s++) {
     cfp::launch_pack(p->stream, p->D, p->VC, n_train, 0, p->B, seed, s, p->norm, p->x, p->tgt);
-    batch_gradient(p, p->B, p->x, p->h1, p->z2, p->tgt, p->dz2, p->part_h, p->part_d, p->part_w);
+    batch_gradient(p, p->B, p->x, p->h1, p->z2, p->tgt, p->dz2, p->along_k, p->part_h, p->part_d, p->part_w);
     // cosine decay of the step size over the run
     const float lr_s = lr * 0.5f * (1.0f + std::cos(3.14159265f * (float)s / (float)steps));
     cfp::launch_adam(p->stream, p->P, p->G, p->M, p->V, ++p->adam_step, lr_s, p->W1b, p->W2b, p->W2Tb);
@@ -258,7 +259,7 @@ extern "C" int cf_pred_eval(cf_pred* p, int first, int n, double* loss, double* 
   for (int c0 = 0; c0 < n; c0 += p->B) {
     const int nb = std::min(p->B, n - c0);
     cfp::launch_pack(p->stream, p->D, p->VC, p->n_crops, first + c0, nb, 0, -1, p->norm, p->x, p->tgt);
-    batch_gradient(p, nb, p->x, p->h1, p->z2, p->tgt, p->dz2, p->part_h, p->part_d, p->part_w);
+    batch_gradient(p, nb, p->x, p->h1, p->z2, p->tgt, p->dz2, p->along_k, p->part_h, p->part_d, p->part_w);
     float g = 0;
     PCHK(p, hipMemcpyAsync(&g, p->G + cfp::NPARAM, 4, hipMemcpyDeviceToHost, p->stream));
     PCHK(p, hipMemcpyAsync(t.data(), p->tgt, (size_t)nb * ni3 * cfp::COUT * 4, hipMemcpyDeviceToHost, p->stream));
@@ -313,21 +314,29 @@ extern "C" int cf_pred_gradient(cf_pred* p, int n, const float* x, const float* 
   const cfp::Vol v = pred_batch_vol(n, VC);
   const long n3 = v.cells(), ni3 = v.inner_cells();
   const cfp::Vol full = cfp::make_vol(n, VC, VC, VC, 0);
-  float *xf = nullptr, *z2 = nullptr, *tg = nullptr, *ph = nullptr, *pd = nullptr, *pw = nullptr;
-  unsigned short *xb = nullptr, *h1 = nullptr, *dz2 = nullptr;
+  // a batch that fits takes the training step's buffers, with the host's floats
+  // in z2, which the forward pass writes after they are rounded
+  const bool own = n <= p->B;
+  float *xf = own ? p->z2 : nullptr, *z2 = xf, *tg = own ? p->tgt : nullptr, *ph = own ? p->part_h : nullptr,
+        *pd = own ? p->part_d : nullptr, *pw = p->part_w;
+  unsigned short *xb = own ? p->x : nullptr, *h1 = own ? p->h1 : nullptr, *dz2 = own ? p->dz2 : nullptr,
+                 *ak = own ? p->along_k : nullptr;
   int rc = CF_OK;
-  if (dalloc(&xf, (size_t)n3 * cfp::CIN) || dalloc(&xb, (size_t)n3 * cfp::CIN) || dalloc(&h1, (size_t)n3 * cfp::CH) ||
-      dalloc(&dz2, (size_t)n3 * cfp::CH) || dalloc(&z2, (size_t)ni3 * cfp::CH) || dalloc(&tg, (size_t)ni3 * cfp::COUT) ||
-      dalloc(&ph, (size_t)((ni3 + 63) / 64) * cfp::HEAD_PART) || dalloc(&pd, (size_t)full.bricks() * cfp::NW1) ||
-      dalloc(&pw, (size_t)p->splits * cfp::NW2)) {
+  if (!own &&
+      (dalloc(&z2, (size_t)ni3 * cfp::CH) || dalloc(&xb, (size_t)n3 * cfp::CIN) || dalloc(&h1, (size_t)n3 * cfp::CH) ||
+       dalloc(&dz2, (size_t)n3 * cfp::CH) || dalloc(&tg, (size_t)ni3 * cfp::COUT) ||
+       dalloc(&ph, (size_t)((ni3 + 63) / 64) * cfp::HEAD_PART) || dalloc(&pd, (size_t)full.bricks() * cfp::NW1) ||
+       dalloc(&ak, (size_t)cfp::along_k_elems(v)))) {
     rc = pfail(p, CF_ERR_HIP, "out of device memory");
   } else {
+    xf = z2;
     hipError_t e = hipMemcpyAsync(xf, x, (size_t)n3 * cfp::CIN * 4, hipMemcpyHostToDevice, p->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(tg, target, (size_t)ni3 * cfp::COUT * 4, hipMemcpyHostToDevice, p->stream);
-    if (e == hipSuccess) e = hipMemsetAsync(dz2, 0, (size_t)n3 * cfp::CH * 2, p->stream);
+    // (the training step's dz2 has its margin zero from the start)
+    if (e == hipSuccess && !own) e = hipMemsetAsync(dz2, 0, (size_t)n3 * cfp::CH * 2, p->stream);
     if (e == hipSuccess) {
       cfp::launch_to_bf16(p->stream, xf, xb, n3 * cfp::CIN);
-      batch_gradient(p, n, xb, h1, z2, tg, dz2, ph, pd, pw);
+      batch_gradient(p, n, xb, h1, z2, tg, dz2, ak, ph, pd, pw);
       e = hipGetLastError();
     }
     float sse = 0;
@@ -338,9 +347,9 @@ extern "C" int cf_pred_gradient(cf_pred* p, int n, const float* x, const float* 
     *loss = sse / (5.0 * (double)ni3);
   }
   (void)hipStreamSynchronize(p->stream);
-  void* ptrs[] = {xf, z2, tg, ph, pd, pw, xb, h1, dz2};
+  void* ptrs[] = {z2, tg, ph, pd, xb, h1, dz2, ak};
   for (void* q : ptrs)
-    if (q) (void)hipFree(q);
+    if (q && !own) (void)hipFree(q);
   return rc;
 }
 
@@ -383,7 +392,7 @@ extern "C" int cf_pred_profile(cf_pred* p, int X, int Y, int Z, double ms[CF_PRE
       (void)hipEventRecord(ev[3], p->stream);
       const int db = cfp::launch_bwd_data(p->stream, bv, p->dz2, p->W2Tb, p->x, p->part_d);
       (void)hipEventRecord(ev[4], p->stream);
-      cfp::launch_bwd_weight(p->stream, bv, p->dz2, p->h1, p->splits, p->part_w);
+      cfp::launch_bwd_weight(p->stream, bv, p->dz2, p->h1, p->splits, p->along_k, p->part_w);
       (void)hipEventRecord(ev[5], p->stream);
       cfp::launch_reduce(p->stream, p->part_h, hb, p->part_d, db, p->part_w, p->splits, p->G);
       (void)hipEventRecord(ev[6], p->stream);

@@ -18,12 +18,12 @@ struct cf_pred {
   cfp::Norm norm{};
   bool have_norm = false;
   // training crops: [cap][VC^3][NDATA]
-  int VC = 16;
+  int VC = 16;  // inner cells x CH >= cells x CIN: z2 can hold a batch of features
   long cap = 0, n_crops = 0;
   float* D = nullptr;
   // one training batch of B crops
   int B = 0, splits = 16;
-  unsigned short *x = nullptr, *h1 = nullptr, *dz2 = nullptr;
+  unsigned short *x = nullptr, *h1 = nullptr, *dz2 = nullptr, *along_k = nullptr;
   float *z2 = nullptr, *tgt = nullptr, *part_h = nullptr, *part_d = nullptr, *part_w = nullptr, *losses = nullptr;
   long losses_cap = 0;
   std::string err;

@@ -20,6 +20,8 @@
 //   D[m = 4 g + q][n = r], q < 4
 #include "cf_predictor.hpp"
 
+#include <type_traits>
+
 namespace cfp {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -29,7 +31,6 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int HI = BI + 2, HJ = BJ + 2, HK = BK + 2, HN = HI * HJ * HK;  // halo brick: 600 cells
 constexpr int AS = CH + 1;   // floats per LDS row of the per-cell epilogue arrays
-constexpr int TS = BCELLS + 8;  // bf16 per LDS row of the transposed tiles of the weight gradient
 static_assert(BCELLS == 256 && BI == 4, "one i-plane of 64 cells per wave, 256 threads");
 static_assert(BCELLS * AS * 4 + BCELLS * CIN * 2 <= HN * CH * 2, "epilogue arrays fit in the tile");
 
@@ -238,73 +239,88 @@ __global__ void __launch_bounds__(256) k_l1(Vol v, const unsigned short* __restr
   }
 }
 
-// loss head, one inner cell per thread: y, dy = inv_norm (y - target),
-// dz2 = (W3^T dy) gelu'(z2) into the dz2 volume; block partials of dW3, db2,
-// db3 and the sum of squared errors
-__global__ void __launch_bounds__(64) k_head(Vol v, const float* __restrict__ z2, const float* __restrict__ target,
-                                             const float* __restrict__ P, float inv_norm,
-                                             unsigned short* __restrict__ dz2, float* __restrict__ part) {
-  __shared__ float aT[64][AS], dzT[64][AS], dyT[64][COUT + 1], lossT[64];
-  const int t = threadIdx.x;
-  const long cell = (long)blockIdx.x * 64 + t;
+// loss head on 64 inner cells per block: y, dy = inv_norm (y - target), dz2 =
+// (W3^T dy) gelu'(z2) into the dz2 volume; block partials of dW3, db2, db3 and
+// the sum of squared errors.  Elementwise work has a channel per lane and 16
+// cells per thread (z2 in 256-byte loads), every sum one thread, in index
+// order.  (One wave a block, a cell a thread, each walking its 64 channels
+// alone, took 89 us for a batch of 32 crops; now 37.)
+__global__ void __launch_bounds__(256) k_head(Vol v, const float* __restrict__ z2, const float* __restrict__ target,
+                                              const float* __restrict__ P, float inv_norm,
+                                              unsigned short* __restrict__ dz2, float* __restrict__ part) {
+  __shared__ float aT[64][AS], dzT[64][AS], dyT[64][COUT + 1], eT[64][COUT + 1];
+  __shared__ long at[64];
+  const int t = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const long cell0 = (long)blockIdx.x * 64;
+  const int n = (int)min(64L, v.inner_cells() - cell0);  // the block's cells
   const float* W3 = P + OFF_W3;
   const float* b3 = P + OFF_B3;
-  float dy[COUT] = {0.f, 0.f, 0.f, 0.f, 0.f};
-  float ls = 0.f;
-  if (cell < v.inner_cells()) {
-    const float* z = z2 + cell * CH;
-    for (int co = 0; co < CH; co++) aT[t][co] = gelu(z[co]);
-    for (int c = 0; c < COUT; c++) {
-      float y = b3[c];
-      for (int co = 0; co < CH; co++) y += W3[c * CH + co] * aT[t][co];
-      const float e = y - target[cell * COUT + c];
-      dy[c] = inv_norm * e;
-      ls += e * e;
-    }
-    long rest = cell;
+  float z[16];
+#pragma unroll
+  for (int m = 0; m < 16; m++) {
+    const int u = 4 * m + w;
+    z[m] = u < n ? z2[(cell0 + u) * CH + t] : 0.f;
+    aT[u][t] = u < n ? gelu(z[m]) : 0.f;
+  }
+  if (w == 0 && t < n) {
+    long rest = cell0 + t;
     const int kk = (int)(rest % v.K);
     rest /= v.K;
     const int jj = (int)(rest % v.J);
     rest /= v.J;
     const int ii = (int)(rest % v.I);
-    const int vol = (int)(rest / v.I);
-    unsigned int* dst = reinterpret_cast<unsigned int*>(dz2 + vcell(v, vol, ii + v.m, jj + v.m, kk + v.m) * CH);
-    for (int co = 0; co < CH; co += 2) {
-      float d2[2];
-      for (int e = 0; e < 2; e++) {
-        float da = 0.f;
-        for (int c = 0; c < COUT; c++) da += W3[c * CH + co + e] * dy[c];
-        d2[e] = da * gelu_grad(z[co + e]);
-        dzT[t][co + e] = d2[e];
-      }
-      dst[co >> 1] = (unsigned)f2bf(d2[0]) | ((unsigned)f2bf(d2[1]) << 16);
-    }
-  } else {
-    for (int co = 0; co < CH; co++) {
-      aT[t][co] = 0.f;
-      dzT[t][co] = 0.f;
-    }
+    at[t] = vcell(v, (int)(rest / v.I), ii + v.m, jj + v.m, kk + v.m) * CH;
   }
-  for (int c = 0; c < COUT; c++) dyT[t][c] = dy[c];
-  lossT[t] = ls;
+  __syncthreads();
+  for (int c = w; c < COUT; c += 4) {
+    float e = 0.f;
+    if (t < n) {
+      float y = b3[c];
+      for (int co = 0; co < CH; co++) y += W3[c * CH + co] * aT[t][co];
+      e = y - target[(cell0 + t) * COUT + c];
+    }
+    eT[t][c] = e;
+    dyT[t][c] = inv_norm * e;
+  }
+  __syncthreads();
+  float w3[COUT];
+#pragma unroll
+  for (int c = 0; c < COUT; c++) w3[c] = W3[c * CH + t];
+#pragma unroll
+  for (int m = 0; m < 16; m++) {
+    const int u = 4 * m + w;
+    float d2 = 0.f;
+    if (u < n) {
+      float da = 0.f;
+#pragma unroll
+      for (int c = 0; c < COUT; c++) da += w3[c] * dyT[u][c];
+      d2 = da * gelu_grad(z[m]);
+      dz2[at[u] + t] = f2bf(d2);
+    }
+    dzT[u][t] = d2;
+  }
   __syncthreads();
   float* pp = part + (long)blockIdx.x * HEAD_PART;
-  for (int c = 0; c < COUT; c++) {
+  for (int c = w; c < COUT; c += 4) {
     float s = 0.f;
     for (int u = 0; u < 64; u++) s += dyT[u][c] * aT[u][t];
     pp[c * CH + t] = s;
   }
-  float s = 0.f;
-  for (int u = 0; u < 64; u++) s += dzT[u][t];
-  pp[NW3 + t] = s;
-  if (t < COUT) {
+  if (w == 1) {
+    float s = 0.f;
+    for (int u = 0; u < 64; u++) s += dzT[u][t];
+    pp[NW3 + t] = s;
+  } else if (w == 2 && t < COUT) {
     float sb = 0.f;
     for (int u = 0; u < 64; u++) sb += dyT[u][t];
     pp[NW3 + NB2 + t] = sb;
-  }
-  if (t == COUT) {
+  } else if (w == 3 && t == 0) {
     float sl = 0.f;
-    for (int u = 0; u < 64; u++) sl += lossT[u];
+    for (int u = 0; u < 64; u++) {
+      float ls = 0.f;
+      for (int c = 0; c < COUT; c++) ls += eT[u][c] * eT[u][c];
+      sl += ls;
+    }
     pp[NW3 + NB2 + NB3] = sl;
   }
 }
@@ -355,57 +371,133 @@ __global__ void __launch_bounds__(256) k_bwd_data(Vol v, const unsigned short* _
   }
 }
 
+// The weight gradient's operands with the cells along k: eight bf16 of one
+// channel at k = m + 8 kb + dk .. + 7 (dk = -1, 0, 1; zeros outside the
+// volume), [dk][row][kb][channel][8] with row = (vol VI + i) VJ + j and a last
+// row of zeros, which rows outside the volume read.  A lane loads its share of
+// an MFMA operand from one 16-byte slot.
+__device__ __forceinline__ long kslot(const Vol& v, long row, int kb) { return (row * v.nbk + kb) * CH * 8; }
+
+// blockIdx.y = 0: h1 into its three copies; 1: dz2 into one.  One row (vol,
+// i, j) per wave, one channel per lane: 128-byte loads, 1 KB stores.  With the
+// shift in the copy no tap has a misaligned operand.
+__global__ void __launch_bounds__(256) k_along_k(Vol v, const unsigned short* __restrict__ h1,
+                                                 const unsigned short* __restrict__ dz2,
+                                                 unsigned short* __restrict__ hT, unsigned short* __restrict__ dT) {
+  const long rows = (long)v.n * v.VI * v.VJ, row = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int ch = threadIdx.x & 63;
+  if (row > rows) return;
+  const bool h = blockIdx.y == 0;
+  const unsigned short* src = (h ? h1 : dz2) + row * v.VK * CH + ch;
+  for (int kb = 0; kb < v.nbk; kb++) {
+    unsigned e[10];
+#pragma unroll
+    for (int q = 0; q < 10; q++) {
+      const int k = v.m + kb * 8 - 1 + q;
+      e[q] = row < rows && k >= 0 && k < v.VK ? src[(long)k * CH] : 0u;
+    }
+    const long o = kslot(v, row, kb) + ch * 8;
+    auto put = [&](unsigned short* dst, auto sh) {
+      constexpr int S = decltype(sh)::value;
+      *reinterpret_cast<u32x4*>(dst + o) = u32x4{e[S] | e[S + 1] << 16, e[S + 2] | e[S + 3] << 16,
+                                                 e[S + 4] | e[S + 5] << 16, e[S + 6] | e[S + 7] << 16};
+    };
+    if (h) {
+      const long copy = kslot(v, rows + 1, 0);
+      put(hT, std::integral_constant<int, 0>{});
+      put(hT + copy, std::integral_constant<int, 1>{});
+      put(hT + 2 * copy, std::integral_constant<int, 2>{});
+    } else {
+      put(dT, std::integral_constant<int, 1>{});
+    }
+  }
+}
+
 // dW2[t][co][ci] = sum over cells of dz2(p)[co] h1(p + o_t)[ci]; block
-// (split s, tap t) walks its share of the inner bricks with both operands
-// transposed in LDS (cells along K), then writes its partial
-__global__ void __launch_bounds__(256) k_bwd_weight(Vol v, const unsigned short* __restrict__ dz2,
-                                                    const unsigned short* __restrict__ h1, int splits,
+// (split s, tap t) walks its share of the inner bricks, then writes its
+// partial.  Both operands come from the copies along k, a wave a 32 x 32 part
+// of the product: four loads for four MFMAs, none through LDS.  (Transposing
+// each brick in LDS for each of the 27 taps, with 128 two-byte stores a thread
+// for 32 MFMAs a wave, took 245 us for a batch of 32 crops; now
+// 88, and 16 for the copies.  What is left is the loads: 128 KB a brick and
+// block through the L1.)
+__global__ void __launch_bounds__(256) k_bwd_weight(Vol v, const unsigned short* __restrict__ dT,
+                                                    const unsigned short* __restrict__ hT, int splits,
                                                     float* __restrict__ part) {
-  __shared__ __attribute__((aligned(16))) unsigned short T1[CH * TS];
-  __shared__ __attribute__((aligned(16))) unsigned short T2[CH * TS];
   const int t = blockIdx.x % 27, s = blockIdx.x / 27;
-  const int di = t / 9 - 1, dj = (t / 3) % 3 - 1, dk = t % 3 - 1;
+  const int di = t / 9 - 1, dj = (t / 3) % 3 - 1, dk = t % 3;
   const long nb = v.bricks(), b0 = nb * s / splits, b1 = nb * (s + 1) / splits;
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, g = l >> 4, r = l & 15;
-  f32x4 acc[4];
+  const int co = 32 * (w >> 1), ci = 32 * (w & 1);
+  const long rows = (long)v.n * v.VI * v.VJ;
+  const unsigned short* hk = hT + dk * kslot(v, rows + 1, 0) + (ci + r) * 8;
+  const unsigned short* dp = dT + (co + r) * 8;
+  f32x4 acc[2][2];
 #pragma unroll
-  for (int nt = 0; nt < 4; nt++) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (long b = b0; b < b1; b++) {
-    int vol, i0, j0, k0;
-    brick_of(v, b, &vol, &i0, &j0, &k0);
-    __syncthreads();  // the previous brick's operands have been read
-    {
-      const int o = threadIdx.x;
-      int ii, jj, kk;
-      cell_of(o, &ii, &jj, &kk);
-      const int i = i0 + ii, j = j0 + jj, k = k0 + kk;
-      const bool in_d = inside(v, i, j, k), in_h = inside(v, i + di, j + dj, k + dk);
-      const u32x4* pd = reinterpret_cast<const u32x4*>(dz2 + (in_d ? vcell(v, vol, i, j, k) * CH : 0));
-      const u32x4* ph = reinterpret_cast<const u32x4*>(h1 + (in_h ? vcell(v, vol, i + di, j + dj, k + dk) * CH : 0));
+  for (int mt = 0; mt < 2; mt++)
 #pragma unroll
-      for (int c = 0; c < 8; c++) {
-        const u32x4 dv = in_d ? pd[c] : u32x4{0u, 0u, 0u, 0u};
-        const u32x4 hv = in_h ? ph[c] : u32x4{0u, 0u, 0u, 0u};
+    for (int nt = 0; nt < 2; nt++) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  int vol, i0, j0, k0;
+  brick_of(v, b0, &vol, &i0, &j0, &k0);
+  auto next = [&]() {  // brick_of(b + 1) without its divisions
+    if ((k0 += BK) < v.m + v.nbk * BK) return;
+    k0 = v.m;
+    if ((j0 += BJ) < v.m + v.nbj * BJ) return;
+    j0 = v.m;
+    if ((i0 += BI) < v.m + v.nbi * BI) return;
+    i0 = v.m;
+    vol++;
+  };
+  constexpr int HC = BCELLS / 32 / 2;  // K = 32 products per half brick
+  struct Half {
+    bf16x8 a[HC][2], b[HC][2];
+  };
+  auto load = [&](int half, Half& f) {
+    const int kb = (k0 - v.m) / BK;
 #pragma unroll
-        for (int e = 0; e < 8; e++) {
-          T1[(c * 8 + e) * TS + o] = (unsigned short)(dv[e >> 1] >> (16 * (e & 1)));
-          T2[(c * 8 + e) * TS + o] = (unsigned short)(hv[e >> 1] >> (16 * (e & 1)));
-        }
+    for (int c = 0; c < HC; c++) {
+      // cells 32 (c + 4 half) + 8 g .. + 7 of the brick: one row of its i, j plane
+      const int o = 4 * (c + HC * half) + g, i = i0 + o / BJ, j = j0 + o % BJ;
+      const bool in_d = i < v.VI && j < v.VJ;
+      const bool in_h = i + di >= 0 && i + di < v.VI && j + dj >= 0 && j + dj < v.VJ;
+      const long row = ((long)vol * v.VI + i) * v.VJ + j;
+      const unsigned short* pd = dp + kslot(v, in_d ? row : rows, kb);
+      const unsigned short* ph = hk + kslot(v, in_h ? row + (long)di * v.VJ + dj : rows, kb);
+#pragma unroll
+      for (int q = 0; q < 2; q++) {
+        f.a[c][q] = ld8(pd + q * 128);
+        f.b[c][q] = ld8(ph + q * 128);
       }
     }
-    __syncthreads();
+  };
+  auto product = [&](const Half& f) {
 #pragma unroll
-    for (int c = 0; c < BCELLS / 32; c++) {
-      const bf16x8 av = ld8(T1 + (16 * w + r) * TS + 32 * c + 8 * g);
+    for (int c = 0; c < HC; c++)
 #pragma unroll
-      for (int nt = 0; nt < 4; nt++) acc[nt] = mma32(av, ld8(T2 + (16 * nt + r) * TS + 32 * c + 8 * g), acc[nt]);
+      for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+        for (int nt = 0; nt < 2; nt++) acc[mt][nt] = mma32(f.a[c][mt], f.b[c][nt], acc[mt][nt]);
+  };
+  if (b0 < b1) {
+    Half f0, f1;
+    load(0, f0);
+    for (long b = b0; b < b1; b++) {
+      load(1, f1);
+      __builtin_amdgcn_sched_barrier(0);  // half a brick's loads stay in flight over the other half's products
+      product(f0);
+      if (b + 1 < b1) next();  // the last turn loads its own brick again
+      load(0, f0);
+      __builtin_amdgcn_sched_barrier(0);
+      product(f1);
     }
   }
   float* pp = part + ((long)s * 27 + t) * (CH * CH);
 #pragma unroll
-  for (int nt = 0; nt < 4; nt++)
+  for (int mt = 0; mt < 2; mt++)
 #pragma unroll
-    for (int q = 0; q < 4; q++) pp[(16 * w + 4 * g + q) * CH + 16 * nt + r] = acc[nt][q];
+    for (int nt = 0; nt < 2; nt++)
+#pragma unroll
+      for (int q = 0; q < 4; q++) pp[(co + 16 * mt + 4 * g + q) * CH + ci + 16 * nt + r] = acc[mt][nt][q];
 }
 
 // the gradient in parameter order (W1, W2, b2, W3, b3) and the summed squared
@@ -682,7 +774,7 @@ void launch_l1(hipStream_t st, const Vol& v, const unsigned short* x, const unsi
 int launch_head(hipStream_t st, const Vol& v, const float* z2, const float* target, const float* P, float inv_norm,
                 unsigned short* dz2, float* part) {
   const int nb = (int)((v.inner_cells() + 63) / 64);
-  hipLaunchKernelGGL(k_head, dim3(nb), dim3(64), 0, st, v, z2, target, P, inv_norm, dz2, part);
+  hipLaunchKernelGGL(k_head, dim3(nb), dim3(256), 0, st, v, z2, target, P, inv_norm, dz2, part);
   return nb;
 }
 
@@ -695,9 +787,14 @@ int launch_bwd_data(hipStream_t st, const Vol& v, const unsigned short* dz2, con
 }
 
 void launch_bwd_weight(hipStream_t st, const Vol& v, const unsigned short* dz2, const unsigned short* h1, int splits,
-                       float* part) {
-  hipLaunchKernelGGL(k_bwd_weight, dim3(27 * splits), dim3(256), 0, st, v, dz2, h1, splits, part);
+                       unsigned short* along_k, float* part) {
+  const long rows = (long)v.n * v.VI * v.VJ;
+  unsigned short* dT = along_k + 3 * (rows + 1) * v.nbk * CH * 8;
+  hipLaunchKernelGGL(k_along_k, dim3((unsigned)(rows / 4 + 1), 2), dim3(256), 0, st, v, h1, dz2, along_k, dT);
+  hipLaunchKernelGGL(k_bwd_weight, dim3(27 * splits), dim3(256), 0, st, v, dT, along_k, splits, part);
 }
+
+long along_k_elems(const Vol& v) { return 4 * ((long)v.n * v.VI * v.VJ + 1) * v.nbk * CH * 8; }
 
 void launch_reduce(hipStream_t st, const float* head_part, int head_blocks, const float* data_part, int data_blocks,
                    const float* w_part, int splits, float* grad) {

@@ -58,9 +58,11 @@ int launch_head(hipStream_t st, const Vol& v, const float* z2, const float* targ
 // [brick][NW1]; returns the brick count
 int launch_bwd_data(hipStream_t st, const Vol& v, const unsigned short* dz2, const unsigned short* W2Tb,
                     const unsigned short* x, float* part);
-// per-split partials of dW2 [split][27][64][64]
+// per-split partials of dW2 [split][27][64][64]; along_k: along_k_elems(v)
+// bf16 of scratch
 void launch_bwd_weight(hipStream_t st, const Vol& v, const unsigned short* dz2, const unsigned short* h1, int splits,
-                       float* part);
+                       unsigned short* along_k, float* part);
+long along_k_elems(const Vol& v);
 // gradient (NPARAM) and loss (at [NPARAM]) from the partials, in a fixed order
 void launch_reduce(hipStream_t st, const float* head_part, int head_blocks, const float* data_part, int data_blocks,
                    const float* w_part, int splits, float* grad);
