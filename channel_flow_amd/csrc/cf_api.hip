@@ -922,13 +922,22 @@ static int finish_iteration(cf_ctx* c, double er[5]) {
 }
 
 // the implicit part of one inner iteration on device-resident fields
+// Where the Jacobi sweeps keep their summary, or null for the general kernel:
+// it needs diagonal metrics, and room in the sweep buffer's scratch, which the
+// ghost layers of the smallest grids exceed (from 16x12x16 it fits).  Per
+// sweep 154 us general at 128x96x128, 106 and a quarter of 40 with the summary.
+static double* jacobi_scratch(const cf_ctx* c) {
+  return diagonal_metrics(c) && cf::jacobi_summary_elems(c->g) <= cf::sweep_scratch_elems(c->g, c->fp32) ? c->Sm
+                                                                                                       : nullptr;
+}
+
 // DPLUSGS on device-resident fields: the same RHS, four Jacobi sweeps, then
 // the update and norms (DPLUSGS.cpp:189-1361)
 static int dplusgs_device(cf_ctx* c, double deltaT, double er[5]) {
   const Geo& g = c->g;
   cf::launch_rhs(c->stream, c->Ui, c->Un, c->Uq, c->Fx, c->Fy, c->Fz, c->vF, c->prof, c->MR, c->NL, g, deltaT,
                  c->p.f_drive);
-  cf::launch_dplusgs(c->stream, c->Ui, c->MR, c->NL, c->NR, c->prof, g, deltaT);
+  cf::launch_dplusgs(c->stream, c->Ui, c->MR, c->NL, c->NR, c->prof, g, deltaT, jacobi_scratch(c));
   double DN = 1. / ((double)c->p.X_out * c->p.Y_out * c->p.Z_out);
   cf::launch_update(c->stream, c->Ui, c->NR, c->prof, c->partial, c->er_dev, g, DN);
   int r = sync(c);
@@ -1180,7 +1189,7 @@ static void enqueue_iteration(cf_ctx* c) {
     // DPLUSGS.cpp:189-1361: the RHS, four Jacobi sweeps, the update and norms
     cf::launch_rhs(c->stream, c->Ui, c->Un, c->Uq, c->Fx, c->Fy, c->Fz, c->vF, c->prof, c->MR, c->NL, g,
                    c->p.deltaT, c->p.f_drive);
-    cf::launch_dplusgs(c->stream, c->Ui, c->MR, c->NL, c->NR, c->prof, g, c->p.deltaT);
+    cf::launch_dplusgs(c->stream, c->Ui, c->MR, c->NL, c->NR, c->prof, g, c->p.deltaT, jacobi_scratch(c));
     const double DN = 1. / ((double)c->p.X_out * c->p.Y_out * c->p.Z_out);
     cf::launch_update(c->stream, c->Ui, c->NR, c->prof, c->partial, c->er_dev, g, DN);
     return;

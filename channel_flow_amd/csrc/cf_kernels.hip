@@ -1437,12 +1437,13 @@ constexpr int LDS_F = 16;
 __device__ __forceinline__ DNb dnb_at(const double* __restrict__ S, long nsk, long p, int d, double n) {
   DNb c;
   const double rho = S[G_RHO * nsk + p];
+  const double rr = rcp_rho(rho);
   c.P = S[G_P * nsk + p];
-  c.T = c.P / rho;
+  c.T = over_rho(c.P, rho, rr);
   c.beta = S[G_BETA * nsk + p];
   c.U = S[(G_UX + 2 * d) * nsk + p];
   c.lam = S[(G_LX + 2 * d) * nsk + p];
-  split_pd_p51(n, c.U, c.beta, rho, rcp_rho(rho), &c.pd, &c.p51);
+  split_pd_p51(n, c.U, c.beta, rho, rr, &c.pd, &c.p51);
   return c;
 }
 
@@ -2333,6 +2334,81 @@ __global__ void __launch_bounds__(256) k_jacobi(const double* __restrict__ Ui, c
   NRout[4 * nf + c] = d51 * (M[0] - LL[0] - UU[0]) + d22 * (M[4] - LL[4] - UU[4]);
 }
 
+// The same sweep for diagonal metrics from the summary (DiagField) of every
+// interior cell, formed once for the four sweeps: a neighbour is then ten
+// loads and one division in place of its primitives, spectral radius and split
+// Jacobian with a dozen divisions and a square root, six times per cell and
+// sweep.  128x96x128: 154 -> 106 us a sweep and 40 us for the summary; the
+// four sweeps read 24 fields each, 60 us of traffic.  S: G_N fields of nf values.
+__global__ void __launch_bounds__(256) k_jacobi_summary(const double* __restrict__ Ui, const double* __restrict__ prof,
+                                                        double* __restrict__ S, Geo g) {
+  const int k = 2 + blockIdx.x * blockDim.x + threadIdx.x;
+  const int j = 2 + blockIdx.y * blockDim.y + threadIdx.y;
+  const int i = 3 + blockIdx.z;
+  if (k > g.nz || j > g.ny) return;
+  const long c = at(g, i, j, k);
+  double u5[5], v[G_N];
+  ld5(Ui, g.nf, c, u5);
+  prep_summary(u5, prof, g, j, v);
+#pragma unroll
+  for (int r = 0; r < G_N; r++) S[r * g.nf + c] = v[r];
+}
+
+constexpr int JAC_JG = 4;  // blocks along j that a walk along i takes with it
+
+__global__ void __launch_bounds__(256) k_jacobi_diag(const double* __restrict__ S, const double* __restrict__ MR,
+                                                     const double* __restrict__ NLin, double* __restrict__ NRout,
+                                                     const double* __restrict__ prof, Geo g, double deltaT) {
+  int bx, by, bz;
+  xcd_block3(&bx, &by, &bz);
+  // grid (k blocks x JAC_JG, i, groups along j): consecutive blocks walk i, so
+  // that the i neighbours' planes of a group are still in the L2 (256x192x256:
+  // 3% of an iteration against whole planes, 1 to 8 blocks within 2%)
+  const int nkb = gridDim.x / JAC_JG;
+  const int k = 2 + (bx % nkb) * blockDim.x + threadIdx.x;
+  const int j = 2 + (bz * JAC_JG + bx / nkb) * blockDim.y + threadIdx.y;
+  const int i = 3 + by;
+  if (k > g.nz || j > g.ny) return;
+  const long nf = g.nf;
+  const long c = at(g, i, j, k);
+  double lo[3][5], hi[3][5];
+  for_each<3>([&](auto d) {
+    constexpr int D = decltype(d)::value;
+    const long st = D == 0 ? g.plane : (D == 1 ? (long)g.Zp : 1L);
+    const bool in_lo = D == 0 ? i - 1 >= 3 : D == 1 ? j - 1 >= 2 : k - 1 >= 2;
+    const bool in_hi = D == 0 ? i + 1 <= g.gend : D == 1 ? j + 1 <= g.ny : k + 1 <= g.nz;
+#pragma unroll
+    for (int v = 0; v < 5; v++) lo[D][v] = hi[D][v] = 0.0;  // ghost neighbours: NL is zero there
+    double N[5];
+    if (in_lo) {
+      const double n = pf(prof, g.Ym, SET_C, 1 + 4 * D, D == 1 ? j - 1 : j);
+      ld5(NLin, nf, c - st, N);
+      lower_diag<D>(dnb_at(S, nf, c - st, D, n), n, N, lo[D]);
+    }
+    if (in_hi) {
+      const double n = pf(prof, g.Ym, SET_C, 1 + 4 * D, D == 1 ? j + 1 : j);
+      ld5(NLin, nf, c + st, N);
+      upper_diag<D>(dnb_at(S, nf, c + st, D, n), n, N, hi[D]);
+    }
+  });
+  double LL[5], UU[5];
+#pragma unroll
+  for (int v = 0; v < 5; v++) {
+    LL[v] = div_rn(lo[0][v], g.dXI, g.rXI) + div_rn(lo[1][v], g.dET, g.rET) + div_rn(lo[2][v], g.dZT, g.rZT);
+    UU[v] = div_rn(hi[0][v], g.dXI, g.rXI) + div_rn(hi[1][v], g.dET, g.rET) + div_rn(hi[2][v], g.dZT, g.rZT);
+  }
+  double d11, d22, d51;
+  diag_dinv<false>(S[G_BETA * nf + c], S[G_RHO * nf + c], S[G_LX * nf + c], S[G_LY * nf + c], S[G_LZ * nf + c], g,
+                   deltaT, &d11, &d22, &d51);
+  double M[5];
+  ld5(MR, nf, c, M);
+  NRout[c] = d11 * (M[0] - LL[0] - UU[0]);
+  NRout[nf + c] = d22 * (M[1] - LL[1] - UU[1]);
+  NRout[2 * nf + c] = d22 * (M[2] - LL[2] - UU[2]);
+  NRout[3 * nf + c] = d22 * (M[3] - LL[3] - UU[3]);
+  NRout[4 * nf + c] = d51 * (M[0] - LL[0] - UU[0]) + d22 * (M[4] - LL[4] - UU[4]);
+}
+
 // Initial iterate of a physical step from the time levels, on the interior:
 // order 1: 2 U^n - U^{n-1}; order 2: 3 U^n - 3 U^{n-1} + U^{n-2}; order 3:
 // 4 U^n - 6 U^{n-1} + 4 U^{n-2} - U^{n-3}.  The reference starts every
@@ -2958,6 +3034,8 @@ long sweep_field_elems(const Geo& g) { return sweep_layout(g).nsk; }
 // float layout has half the bytes, and what follows it is kept)
 long sweep_scratch_elems(const Geo& g, bool fp32) { return (G_N + 5) * sweep_layout(g).nsk / (fp32 ? 2 : 1); }
 
+long jacobi_summary_elems(const Geo& g) { return G_N * g.nf; }
+
 long sweep_buffer_elems(const Geo& g) {
   const Sk q = sweep_layout(g);
   return (G_N + 15) * q.nsk + 2 * ho_at(q, q.ntiles, 0, 0);
@@ -3102,14 +3180,18 @@ void launch_copy_interior(hipStream_t st, const double* src, double* dst, const 
 }
 
 void launch_dplusgs(hipStream_t st, const double* Ui, const double* MR, double* NL, double* NR, const double* prof,
-                    const Geo& g, double deltaT) {
+                    const Geo& g, double deltaT, double* S) {
   dim3 blk(64, 4);
   dim3 gr = box_grid(g.nz - 1, g.ny - 1, g.gend - 2, blk);
+  if (S) hipLaunchKernelGGL(k_jacobi_summary, gr, blk, 0, st, Ui, prof, S, g);
   // four sweeps, ping-pong NL -> NR -> NL -> NR -> NL; both end with the last
   for (int sweep = 0; sweep < 4; sweep++) {
     const double* in = (sweep & 1) ? NR : NL;
     double* out = (sweep & 1) ? NL : NR;
-    hipLaunchKernelGGL(k_jacobi, gr, blk, 0, st, Ui, MR, in, out, prof, g, deltaT);
+    if (S)
+      hipLaunchKernelGGL(k_jacobi_diag, dim3(gr.x * JAC_JG, gr.z, (gr.y + JAC_JG - 1) / JAC_JG), blk, 0, st, S, MR, in, out, prof, g, deltaT);
+    else
+      hipLaunchKernelGGL(k_jacobi, gr, blk, 0, st, Ui, MR, in, out, prof, g, deltaT);
   }
   launch_copy_interior(st, NL, NR, g);
 }

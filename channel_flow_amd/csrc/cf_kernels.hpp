@@ -78,8 +78,10 @@ void launch_sweeps_planes(hipStream_t st, const double* Ui, const double* MR, do
                           const hipEvent_t* marks = nullptr);
 // DPLUSGS: four point-Jacobi sweeps from NL (= D^-1 MR); NL and NR both end
 // with the last sweep's values (ghosts of both must be zero)
+// (S: jacobi_summary_elems doubles of scratch for diagonal metrics, or null)
+long jacobi_summary_elems(const Geo& g);
 void launch_dplusgs(hipStream_t st, const double* Ui, const double* MR, double* NL, double* NR, const double* prof,
-                    const Geo& g, double deltaT);
+                    const Geo& g, double deltaT, double* S);
 void launch_copy_interior(hipStream_t st, const double* src, double* dst, const Geo& g);
 // U_ <- 2 U^n - U^{n-1} (order 1), 3 U^n - 3 U^{n-1} + U^{n-2} (order 2) or
 // 4 U^n - 6 U^{n-1} + 4 U^{n-2} - U^{n-3} (order 3, U3 = U^{n-3}), interior
