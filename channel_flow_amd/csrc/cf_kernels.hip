@@ -167,8 +167,8 @@ __global__ void __launch_bounds__(256) k_flux_zs(const double* __restrict__ U, c
 // face ahead) where a thread per face loads up to six.  16 faces per
 // thread measured faster than 8 and equal to 32 at 256x192x256.
 constexpr int FC = 16;
-// at least 3 waves per SIMD: x takes 126 VGPRs (4 waves), y 144 (forcing
-// 4 waves spills y and took 3% longer)
+// at least 3 waves per SIMD: x takes 126 VGPRs (4 waves), y 129 (forcing 4
+// took y from 318 to 350 us)
 constexpr int FLUX_COL_WAVES = 3;
 
 template <int DIR>
