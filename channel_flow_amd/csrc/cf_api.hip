@@ -924,8 +924,8 @@ static int finish_iteration(cf_ctx* c, double er[5]) {
 // the implicit part of one inner iteration on device-resident fields
 // Where the Jacobi sweeps keep their summary, or null for the general kernel:
 // it needs diagonal metrics, and room in the sweep buffer's scratch, which the
-// ghost layers of the smallest grids exceed (from 16x12x16 it fits).  Per
-// sweep 154 us general at 128x96x128, 106 and a quarter of 40 with the summary.
+// ghost layers of thin grids exceed (8x8x64).  Per sweep at 128x96x128: 154 us
+// general, 100 and a quarter of 34 with the summary.
 static double* jacobi_scratch(const cf_ctx* c) {
   return diagonal_metrics(c) && cf::jacobi_summary_elems(c->g) <= cf::sweep_scratch_elems(c->g, c->fp32) ? c->Sm
                                                                                                        : nullptr;

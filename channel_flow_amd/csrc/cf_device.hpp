@@ -321,11 +321,17 @@ __device__ __forceinline__ PState prim_dt(double U1, double U2, double U3, doubl
   return s;
 }
 
+// spectral radius of one direction: U the contravariant velocity, C = K P / rho,
+// nn the metric row's square
+__device__ __forceinline__ double lambda_of(double U, double beta, double C, double nn) {
+  double S = sqrt(U * U * (beta - 1) * (beta - 1) + 4 * beta * C * nn);
+  return ((beta + 1) * fabs(U) + S) / 2;
+}
+
 __device__ __forceinline__ double lambda_dir(const PState& s, double n0, double n1, double n2, double* Uc) {
   double U = n0 * s.u + n1 * s.v + n2 * s.w;
-  double S = sqrt(U * U * (s.beta - 1) * (s.beta - 1) + 4 * s.beta * s.C * (n0 * n0 + n1 * n1 + n2 * n2));
   *Uc = U;
-  return ((s.beta + 1) * fabs(U) + S) / 2;
+  return lambda_of(U, s.beta, s.C, n0 * n0 + n1 * n1 + n2 * n2);
 }
 
 // D^-1 = {d11, d22 (= d33 = d44 = d55), d51}, Dual_time_stepping.cpp:464-489,

@@ -2334,12 +2334,14 @@ __global__ void __launch_bounds__(256) k_jacobi(const double* __restrict__ Ui, c
   NRout[4 * nf + c] = d51 * (M[0] - LL[0] - UU[0]) + d22 * (M[4] - LL[4] - UU[4]);
 }
 
-// The same sweep for diagonal metrics from the summary (DiagField) of every
-// interior cell, formed once for the four sweeps: a neighbour is then ten
-// loads and one division in place of its primitives, spectral radius and split
-// Jacobian with a dozen divisions and a square root, six times per cell and
-// sweep.  128x96x128: 154 -> 106 us a sweep and 40 us for the summary; the
-// four sweeps read 24 fields each, 60 us of traffic.  S: G_N fields of nf values.
+// The same sweep for diagonal metrics from a summary of every interior cell,
+// formed once for the four sweeps: P, beta, rho and the three contravariant
+// velocities.  A neighbour is then nine loads, one division and one square root
+// in place of its primitives and split Jacobian with a dozen divisions, six
+// times per cell and sweep.  Bound by memory: the six neighbours' fields miss
+// the L2 by half, so stored spectral radii (nine fields) cost more than their
+// roots, 106 us a sweep.  128x96x128: 154 -> 100 us a sweep, and 34 for the
+// summary.  S: jacobi_summary_elems doubles.
 __global__ void __launch_bounds__(256) k_jacobi_summary(const double* __restrict__ Ui, const double* __restrict__ prof,
                                                         double* __restrict__ S, Geo g) {
   const int k = 2 + blockIdx.x * blockDim.x + threadIdx.x;
@@ -2350,8 +2352,25 @@ __global__ void __launch_bounds__(256) k_jacobi_summary(const double* __restrict
   double u5[5], v[G_N];
   ld5(Ui, g.nf, c, u5);
   prep_summary(u5, prof, g, j, v);
+  S[c] = v[G_P];
+  S[g.nf + c] = v[G_BETA];
+  S[2 * g.nf + c] = v[G_RHO];
 #pragma unroll
-  for (int r = 0; r < G_N; r++) S[r * g.nf + c] = v[r];
+  for (int d = 0; d < 3; d++) S[(3 + d) * g.nf + c] = v[G_UX + 2 * d];
+}
+
+// neighbour p along direction d from that summary; n: the diagonal metric entry at its j
+__device__ __forceinline__ DNb jacobi_nb(const double* __restrict__ S, long nf, long p, int d, double n) {
+  DNb c;
+  const double rho = S[2 * nf + p];
+  const double rr = rcp_rho(rho);
+  c.P = S[p];
+  c.T = over_rho(c.P, rho, rr);
+  c.beta = S[nf + p];
+  c.U = S[(3 + d) * nf + p];
+  c.lam = lambda_of(c.U, c.beta, over_rho(KG * c.P, rho, rr), n * n);
+  split_pd_p51(n, c.U, c.beta, rho, rr, &c.pd, &c.p51);
+  return c;
 }
 
 constexpr int JAC_JG = 4;  // blocks along j that a walk along i takes with it
@@ -2383,12 +2402,12 @@ __global__ void __launch_bounds__(256) k_jacobi_diag(const double* __restrict__ 
     if (in_lo) {
       const double n = pf(prof, g.Ym, SET_C, 1 + 4 * D, D == 1 ? j - 1 : j);
       ld5(NLin, nf, c - st, N);
-      lower_diag<D>(dnb_at(S, nf, c - st, D, n), n, N, lo[D]);
+      lower_diag<D>(jacobi_nb(S, nf, c - st, D, n), n, N, lo[D]);
     }
     if (in_hi) {
       const double n = pf(prof, g.Ym, SET_C, 1 + 4 * D, D == 1 ? j + 1 : j);
       ld5(NLin, nf, c + st, N);
-      upper_diag<D>(dnb_at(S, nf, c + st, D, n), n, N, hi[D]);
+      upper_diag<D>(jacobi_nb(S, nf, c + st, D, n), n, N, hi[D]);
     }
   });
   double LL[5], UU[5];
@@ -2398,8 +2417,14 @@ __global__ void __launch_bounds__(256) k_jacobi_diag(const double* __restrict__ 
     UU[v] = div_rn(hi[0][v], g.dXI, g.rXI) + div_rn(hi[1][v], g.dET, g.rET) + div_rn(hi[2][v], g.dZT, g.rZT);
   }
   double d11, d22, d51;
-  diag_dinv<false>(S[G_BETA * nf + c], S[G_RHO * nf + c], S[G_LX * nf + c], S[G_LY * nf + c], S[G_LZ * nf + c], g,
-                   deltaT, &d11, &d22, &d51);
+  const double beta = S[nf + c], rho = S[2 * nf + c], C = over_rho(KG * S[c], rho, rcp_rho(rho));
+  double lam[3];
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    const double n = pf(prof, g.Ym, SET_C, 1 + 4 * d, j);
+    lam[d] = lambda_of(S[(3 + d) * nf + c], beta, C, n * n);
+  }
+  diag_dinv<false>(beta, rho, lam[0], lam[1], lam[2], g, deltaT, &d11, &d22, &d51);
   double M[5];
   ld5(MR, nf, c, M);
   NRout[c] = d11 * (M[0] - LL[0] - UU[0]);
@@ -3034,7 +3059,7 @@ long sweep_field_elems(const Geo& g) { return sweep_layout(g).nsk; }
 // float layout has half the bytes, and what follows it is kept)
 long sweep_scratch_elems(const Geo& g, bool fp32) { return (G_N + 5) * sweep_layout(g).nsk / (fp32 ? 2 : 1); }
 
-long jacobi_summary_elems(const Geo& g) { return G_N * g.nf; }
+long jacobi_summary_elems(const Geo& g) { return 6 * g.nf; }
 
 long sweep_buffer_elems(const Geo& g) {
   const Sk q = sweep_layout(g);

@@ -1,6 +1,6 @@
 """The DPLUSGS Jacobi sweeps on grids at the edges of their blocks (64 x 4
 cells, four blocks along j walking i) and on both sides of the rule that picks
-the kernel: the summary of the smallest grid does not fit the sweep buffer's
+the kernel: the summary of a thin grid (8x8x64) does not fit the sweep buffer's
 scratch and takes the general one.  The oracle adds in the same order, so the
 iterate agrees bit for bit, the norms to 1e-12."""
 import numpy as np
@@ -17,7 +17,7 @@ def _need_gpu():
         pytest.fail("no GPU visible: the gpu tests must run on an MI355X")
 
 
-@pytest.mark.parametrize("grid", [(8, 8, 8), (9, 17, 11), (10, 24, 66), (33, 9, 24)])
+@pytest.mark.parametrize("grid", [(8, 8, 8), (8, 8, 64), (9, 17, 11), (10, 24, 66), (33, 9, 24)])
 def test_gpu_jacobi_sweeps_match_oracle(grid):
     from oracle import oracle as O
     from channel_flow_amd.config import ChannelConfig, FlowParams, poiseuille_state
