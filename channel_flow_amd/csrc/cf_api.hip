@@ -1133,6 +1133,15 @@ extern "C" int cf_read_state(cf_ctx* c, double* const Qn[5], double* const Qnm1[
   return CF_OK;
 }
 
+// Whether the iteration is replayed as a graph: with the pipelined sweeps or
+// the Jacobi sweeps, whose captures are tested.  A process that captured the
+// per-hyperplane and the single-wave schedules ended in a segmentation fault on
+// the host, of unknown cause: these run as eager launches, which give the same
+// bits.
+static bool replays_graph(const cf_ctx* c) {
+  return c->use_graph && (c->solver == 1 || (c->schedule == 0 && effective_schedule(c) == 0));
+}
+
 // Whether the stencils run on four streams.  The fork and join cost seven event
 // calls eagerly (about 30 us: 16x12x16 124 us an iteration on one stream, 155
 // on four; 64^3 337 and 357; 128x96x128 855 and 871; 256x192x256 4301 and
@@ -1140,7 +1149,7 @@ extern "C" int cf_read_state(cf_ctx* c, double* const Qn[5], double* const Qnm1[
 // 4311 and 4246).
 static bool fork_pays(const cf_ctx* c) {
   const long cells = (long)c->p.X_out * c->p.Y_out * c->p.Z_out;
-  return cells >= (c->use_graph ? 150000 : 4000000);
+  return cells >= (replays_graph(c) ? 150000 : 4000000);
 }
 
 // Everything one inner iteration of the device state launches: kernels
@@ -1236,7 +1245,7 @@ extern "C" int cf_inner_iteration(cf_ctx* c, double er[5]) {
   if (!c || !er) return CF_ERR_ARG;
   if (!c->have_state) return fail(c, CF_ERR_STATE, "no state loaded");
   if (int r = prepare_iteration(c)) return r;
-  if (c->use_graph) {
+  if (replays_graph(c)) {
     if (int r = launch_graph(c)) return r;
   } else {
     enqueue_iteration(c);

@@ -465,7 +465,8 @@ class Solver:
         self._chk(self.lib.cf_set_spin_limit(self._h, int(polls)))
 
     def set_graph(self, enabled: bool = True):
-        """Replay each inner iteration's kernels as a captured hipGraph."""
+        """Replay each inner iteration's kernels as a captured hipGraph (sweep
+        schedule 0 with diagonal metrics, and DPLUSGS; others launch eagerly)."""
         self._chk(self.lib.cf_set_graph(self._h, int(bool(enabled))))
 
     def set_concurrent_stencils(self, enabled: bool = True):

@@ -326,7 +326,10 @@ int cf_set_spin_limit(cf_ctx* ctx, long long polls);
  * the kernels of one inner iteration as a hipGraph on the context's stream,
  * captured on first use and again when the fields, schedules, precision or
  * parameters it was captured with change; the results are the same bits as
- * the launches issued one by one.  No counterpart in the reference. */
+ * the launches issued one by one.  Only the pipelined sweeps (schedule 0 with
+ * diagonal metrics) and DPLUSGS are captured: with the sweep schedules 1 and
+ * 2, and with metrics that are not diagonal, the launches stay one by one.
+ * No counterpart in the reference. */
 int cf_set_graph(cf_ctx* ctx, int enabled);
 /* Number of graph captures made so far. */
 int cf_graph_builds(cf_ctx* ctx, long long* builds);
