@@ -94,14 +94,17 @@ __host__ __device__ __forceinline__ double rcp_checked(double d) {
   return fabs(e) <= 0x1p-54 ? r : 0.0;
 }
 
-// x/d for any normal divisor d, with r = RN(1/d) as the division gives it:
-// one correction more than div_const.  q1 is x/d with an error of a few 2^-105
-// before its own rounding, so it is within one ulp whatever r's own error, its
-// remainder is exact and Markstein's theorem makes the result the correctly
-// rounded x/d, sign of a zero quotient included: the same bits as x / d while
-// the quotient and x times 2^-53 stay in the normal range.  Five operations
-// where the division takes about twelve: it pays where d has several
-// dividends.
+// x/d for any divisor d whose reciprocal r = RN(1/d) is normal, r as the
+// division gives it: one correction more than div_const.  q1 is x/d with an
+// error of a few 2^-105 before its own rounding, so it is within one ulp
+// whatever r's own error, its remainder is exact and Markstein's theorem makes
+// the result the correctly rounded x/d (for d > 0 the sign of a zero quotient
+// included): the same bits as x / d while the quotient and x times 2^-53 stay
+// in the normal range.  Below that the last bit may differ.  Where the
+// division overflows, or x, d or r is not finite, the result may be NaN and is
+// never another value: whoever returns such quotients to a caller looks for
+// NaN and divides.  Five operations where the division takes about twelve: it
+// pays where d has several dividends.
 __device__ __forceinline__ double div_rn(double x, double d, double r) {
   const double q0 = x * r;
   const double q1 = fma(-fma(q0, d, -x), r, q0);
@@ -238,38 +241,44 @@ __device__ __forceinline__ void reconstruct(int r, const double (&u)[5][6], cons
 // rJf, rin: RN(1/Jf), RN(1/insqr).  Quotients with a common divisor share its
 // reciprocal (div_rn, the same bits): a face has 25 divisions, of which 20 have
 // one of five divisors, and a division is about twelve instructions.
+// Every quotient reaches F, so where one of them was out of div_rn's range (an
+// infinite operand, a zero divisor, an overflow) F holds a NaN: the caller then
+// forms the face again with plain divisions (PLAIN).
+template <bool PLAIN>
 __device__ __forceinline__ void roe_flux(const double L[5], const double Rr[5], const double n[3], const double nt[4],
                                          double Jf, double rJf, double rin, bool energy_norm, bool wall,
                                          double F[5]) {
+  auto quot = [](double x, double d, double r) { return PLAIN ? x / d : div_rn(x, d, r); };
+  auto over_kg1 = [](double x) { return PLAIN ? x / (KG - 1) : div_const(x, KG - 1, RKG); };
   const double insqr = nt[0], N0 = nt[1], N1 = nt[2], N2 = nt[3];
   const double _rho = L[0], _r = 1.0 / _rho;
-  double _u = div_rn(L[1], _rho, _r), _v = div_rn(L[2], _rho, _r), _w = div_rn(L[3], _rho, _r);
+  double _u = quot(L[1], _rho, _r), _v = quot(L[2], _rho, _r), _w = quot(L[3], _rho, _r);
   double _U = n[0] * _u + n[1] * _v + n[2] * _w;
   double _VV = _u * _u + _v * _v + _w * _w;
   double _P = (L[4] - 0.5 * _rho * _VV) * (KG - 1);
-  double _C = div_rn(KG * _P, _rho, _r);
-  double _H = 0.5 * _VV + div_const(_C, KG - 1, RKG);
+  double _C = quot(KG * _P, _rho, _r);
+  double _H = 0.5 * _VV + over_kg1(_C);
   const double rho_ = Rr[0], r_ = 1.0 / rho_;
-  double u_ = div_rn(Rr[1], rho_, r_), v_ = div_rn(Rr[2], rho_, r_), w_ = div_rn(Rr[3], rho_, r_);
+  double u_ = quot(Rr[1], rho_, r_), v_ = quot(Rr[2], rho_, r_), w_ = quot(Rr[3], rho_, r_);
   double U_ = n[0] * u_ + n[1] * v_ + n[2] * w_;
   double VV_ = u_ * u_ + v_ * v_ + w_ * w_;
   double P_ = (Rr[4] - 0.5 * rho_ * VV_) * (KG - 1);
-  double C_ = div_rn(KG * P_, rho_, r_);
-  double H_ = 0.5 * VV_ + div_const(C_, KG - 1, RKG);
+  double C_ = quot(KG * P_, rho_, r_);
+  double H_ = 0.5 * VV_ + over_kg1(C_);
   const double t5 = sqrt(_rho), t6 = sqrt(rho_), t4 = t5 + t6, rt = 1.0 / t4;
   double rho = sqrt(_rho * rho_);
-  double u = div_rn(t5 * _u + t6 * u_, t4, rt);
-  double v = div_rn(t5 * _v + t6 * v_, t4, rt);
-  double w = div_rn(t5 * _w + t6 * w_, t4, rt);
-  double U = div_rn(t5 * _U + t6 * U_, t4, rt);
+  double u = quot(t5 * _u + t6 * u_, t4, rt);
+  double v = quot(t5 * _v + t6 * v_, t4, rt);
+  double w = quot(t5 * _w + t6 * w_, t4, rt);
+  double U = quot(t5 * _U + t6 * U_, t4, rt);
   double VV = u * u + v * v + w * w;
-  double H = div_rn(t5 * _H + t6 * H_, t4, rt);
+  double H = quot(t5 * _H + t6 * H_, t4, rt);
   double C = (H - 0.5 * VV) * (KG - 1);
   double dU1 = rho_ - _rho;
   double dU2 = rho_ * u_ - _rho * _u;
   double dU3 = rho_ * v_ - _rho * _v;
   double dU4 = rho_ * w_ - _rho * _w;
-  double dU5 = (div_const(P_, KG - 1, RKG) + 0.5 * rho_ * VV_) - (div_const(_P, KG - 1, RKG) + 0.5 * _rho * _VV);
+  double dU5 = (over_kg1(P_) + 0.5 * rho_ * VV_) - (over_kg1(_P) + 0.5 * _rho * _VV);
   double S = sqrt(C);
   double temp1 = (P_ - _P) / rho / C;
   double temp2 = U * insqr / S * (U_ - _U) * insqr;
@@ -284,16 +293,16 @@ __device__ __forceinline__ void roe_flux(const double L[5], const double Rr[5], 
   if (wall) {
     F[0] = 0;
     F[1] = 0;
-    F[2] = div_rn(0.5 * (n[1] * (_P + P_) - div_rn(Fav3, insqr, rin)), Jf, rJf);
+    F[2] = quot(0.5 * (n[1] * (_P + P_) - quot(Fav3, insqr, rin)), Jf, rJf);
     F[3] = 0;
     F[4] = 0;
     return;
   }
-  F[0] = div_rn(0.5 * ((_rho * _U + rho_ * U_) - div_rn(Fav1, insqr, rin)), Jf, rJf);
-  F[1] = div_rn(0.5 * ((_rho * _u * _U + rho_ * u_ * U_ + n[0] * (_P + P_)) - div_rn(Fav2, insqr, rin)), Jf, rJf);
-  F[2] = div_rn(0.5 * ((_rho * _v * _U + rho_ * v_ * U_ + n[1] * (_P + P_)) - div_rn(Fav3, insqr, rin)), Jf, rJf);
-  F[3] = div_rn(0.5 * ((_rho * _w * _U + rho_ * w_ * U_ + n[2] * (_P + P_)) - div_rn(Fav4, insqr, rin)), Jf, rJf);
-  F[4] = div_rn(0.5 * ((_U * (3.5 * _P + 0.5 * _rho * _VV) + U_ * (3.5 * P_ + 0.5 * rho_ * VV_)) - div_rn(Fav5, insqr, rin)),
+  F[0] = quot(0.5 * ((_rho * _U + rho_ * U_) - quot(Fav1, insqr, rin)), Jf, rJf);
+  F[1] = quot(0.5 * ((_rho * _u * _U + rho_ * u_ * U_ + n[0] * (_P + P_)) - quot(Fav2, insqr, rin)), Jf, rJf);
+  F[2] = quot(0.5 * ((_rho * _v * _U + rho_ * v_ * U_ + n[1] * (_P + P_)) - quot(Fav3, insqr, rin)), Jf, rJf);
+  F[3] = quot(0.5 * ((_rho * _w * _U + rho_ * w_ * U_ + n[2] * (_P + P_)) - quot(Fav4, insqr, rin)), Jf, rJf);
+  F[4] = quot(0.5 * ((_U * (3.5 * _P + 0.5 * _rho * _VV) + U_ * (3.5 * P_ + 0.5 * rho_ * VV_)) - quot(Fav5, insqr, rin)),
                   Jf, rJf);
 }
 
@@ -410,7 +419,10 @@ enum DiagField : int {
 // x / rho and x / K: correctly rounded in FP64, through the reciprocals; in
 // the FP32 sweeps, products with the hardware reciprocal (1 ulp) and with 1/K,
 // which the inexact inner solve tolerates.  rr = rcp_rho(rho), shared by the
-// quotients of one cell.
+// quotients of one cell.  Infinite operands, and a rho below 2^-1024, whose
+// reciprocal overflows, give NaN; the iteration then returns
+// CF_ERR_NONFINITE, as it does for any state that is not finite (a check of
+// every cell's quotients here took 64^3 from 7.28 to 7.55 ms a step).
 constexpr double RK = 1.0 / KG;  // |RK KG - 1| = 2^-54.4 meets div_const's bound
 __device__ __forceinline__ double over_rho(double x, double rho, double rr) { return div_rn(x, rho, rr); }
 __device__ __forceinline__ float over_rho(float x, float, float rr) { return x * rr; }
@@ -555,6 +567,15 @@ __device__ __forceinline__ Prim prim_visc(double U1, double U2, double U3, doubl
   double VV = q.U * q.U + q.V * q.V + q.W * q.W;
   double P = (U5 - 0.5 * rho * VV) * (KG - 1) * J;
   q.T = P / (rho * RG) / J;
+  if (__builtin_expect(q.T != q.T, 0)) {
+    // an operand outside div_rn's range leaves NaN in U, V or W and so in T
+    q.U = U2 / rho;
+    q.V = U3 / rho;
+    q.W = U4 / rho;
+    VV = q.U * q.U + q.V * q.V + q.W * q.W;
+    P = (U5 - 0.5 * rho * VV) * (KG - 1) * J;
+    q.T = P / (rho * RG) / J;
+  }
   return q;
 }
 

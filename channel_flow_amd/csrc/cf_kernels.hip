@@ -94,10 +94,11 @@ __global__ void __launch_bounds__(256) k_ghosts(double* __restrict__ U, const do
 // ---------------------------------------------------------------------------
 // Face f along DIR of the column (i, j, k) (the cell f along the direction):
 // u[v][t] holds U_ of cells f-2 .. f+3 (t = cell - f + 2); each recipe reads
-// only its own cells.
-template <int DIR>
-__device__ __forceinline__ void flux_face(const double (&u)[5][6], int f, int i, int j, int k,
-                                          const double* __restrict__ prof, double* __restrict__ F, const Geo& g) {
+// only its own cells.  Returns the sum of the five outputs, which is NaN where
+// one of them is; PLAIN as in roe_flux.
+template <int DIR, bool PLAIN>
+__device__ __forceinline__ double flux_face(const double (&u)[5][6], int f, int i, int j, int k,
+                                            const double* __restrict__ prof, double* __restrict__ F, const Geo& g) {
   int rl = recipe_left(DIR, f, g.gend, g.ny, g.nz);
   int rr = recipe_right(DIR, f, g.gend, g.ny, g.nz);
   // 1/sum(w/J) varies with j only: with the cell's j along x and z, with the
@@ -119,9 +120,24 @@ __device__ __forceinline__ void flux_face(const double (&u)[5][6], int f, int i,
   double Jf = pf(prof, g.Ym, set, 0, jp);
   bool wall = DIR == 1 && (f == 1 || f == g.ny);
   const double rJf = prow(prof, g.Ym, FT_RCP + 2 * DIR, jp), rin = prow(prof, g.Ym, FT_RCP + 2 * DIR + 1, jp);
-  roe_flux(L, R, n, nt, Jf, rJf, rin, DIR == 1, wall, out);
+  roe_flux<PLAIN>(L, R, n, nt, Jf, rJf, rin, DIR == 1, wall, out);
 #pragma unroll
   for (int v = 0; v < 5; v++) F[v * g.nf + o] = out[v];
+  return out[0] + out[1] + out[2] + out[3] + out[4];
+}
+
+// v, as a value the compiler knows nothing of (uniform; per lane): what a rare
+// path forms from it is not kept in registers along the usual one (Flux_X 127
+// VGPRs and four waves per SIMD, 132 and three without this)
+template <class T>
+__device__ __forceinline__ T anew_s(T v) {
+  asm volatile("" : "+s"(v));
+  return v;
+}
+template <class T>
+__device__ __forceinline__ T anew_v(T v) {
+  asm volatile("" : "+v"(v));
+  return v;
 }
 
 // threadIdx.y of a block 64 threads wide: one wave per row, so the value is
@@ -138,7 +154,7 @@ __global__ void __launch_bounds__(256) k_flux_zs(const double* __restrict__ U, c
                                                  double* __restrict__ F, Geo g) {
   static_assert(DIR == 2, "faces along k");
   __shared__ double S[4][5][72];
-  const int tx = threadIdx.x, ty = wave_row();  // j's profiles in scalar registers: 84 -> 76 VGPRs
+  const int tx = threadIdx.x, ty = wave_row();  // j's profiles in scalar registers: 80 VGPRs, six waves per SIMD
   const int f0 = 1 + blockIdx.x * 64;
   const int j = 2 + blockIdx.y * 4 + ty, i = 3 + blockIdx.z;
   const bool row = j <= g.ny;
@@ -154,11 +170,20 @@ __global__ void __launch_bounds__(256) k_flux_zs(const double* __restrict__ U, c
   const int f = f0 + tx;
   if (!row || f > g.nz) return;
   double u[5][6];
+  auto cells = [&](int x) {
 #pragma unroll
-  for (int t = 0; t < 6; t++)
+    for (int t = 0; t < 6; t++)
 #pragma unroll
-    for (int v = 0; v < 5; v++) u[v][t] = S[ty][v][tx + t];
-  flux_face<DIR>(u, f, i, j, f, prof, F, g);
+      for (int v = 0; v < 5; v++) u[v][t] = S[ty][v][x + t];
+  };
+  cells(tx);
+  const double s = flux_face<DIR, false>(u, f, i, j, f, prof, F, g);
+  if (__builtin_expect(s != s, 0)) {  // with plain divisions, from the cells again
+    const double* const pr = anew_s(prof);
+    const int x = anew_v(tx);
+    cells(x);
+    flux_face<DIR, true>(u, f0 + x, i, j, f0 + x, pr, anew_s(F), g);
+  }
 }
 
 // Flux_X and Flux_Y with one thread per column of faces: lanes run along k
@@ -167,7 +192,7 @@ __global__ void __launch_bounds__(256) k_flux_zs(const double* __restrict__ U, c
 // face ahead) where a thread per face loads up to six.  16 faces per
 // thread measured faster than 8 and equal to 32 at 256x192x256.
 constexpr int FC = 16;
-// at least 3 waves per SIMD: x takes 126 VGPRs (4 waves), y 129 (forcing 4
+// at least 3 waves per SIMD: x takes 127 VGPRs (4 waves), y 132 (forcing 4
 // took y from 318 to 350 us)
 constexpr int FLUX_COL_WAVES = 3;
 
@@ -193,23 +218,38 @@ __global__ void __launch_bounds__(256, FLUX_COL_WAVES) k_flux_col(const double* 
     return DIR == 0 ? at(g, c, j, k) : at(g, i, c, k);
   };
   double u[5][6];
+  auto cells = [&](int f) {
 #pragma unroll
-  for (int t = 0; t < 6; t++) {
-    const long p = cell(f0 - 2 + t);
+    for (int t = 0; t < 6; t++) {
+      const long p = cell(f - 2 + t);
 #pragma unroll
-    for (int v = 0; v < 5; v++) u[v][t] = U[v * g.nf + p];
-  }
+      for (int v = 0; v < 5; v++) u[v][t] = U[v * g.nf + p];
+    }
+  };
+  bool again = false;
+  cells(f0);
   for (int f = f0; f <= f1; f++) {
     double nx[5];
     const long p = cell(f + 4);
 #pragma unroll
     for (int v = 0; v < 5; v++) nx[v] = U[v * g.nf + p];
-    flux_face<DIR>(u, f, DIR == 0 ? f : i, DIR == 0 ? j : f, k, prof, F, g);
+    const double s = flux_face<DIR, false>(u, f, DIR == 0 ? f : i, DIR == 0 ? j : f, k, prof, F, g);
+    again |= s != s;
 #pragma unroll
     for (int v = 0; v < 5; v++) {
 #pragma unroll
       for (int t = 0; t < 5; t++) u[v][t] = u[v][t + 1];
       u[v][5] = nx[v];
+    }
+  }
+  // a NaN among the run's outputs: all of them again with plain divisions,
+  // after the run, where nothing else is held in registers
+  if (__builtin_expect(again, 0)) {
+    const double* const pr = anew_s(prof);
+    const int kk = anew_v(k);
+    for (int f = f0; f <= f1; f++) {
+      cells(f);
+      flux_face<DIR, true>(u, f, DIR == 0 ? f : i, DIR == 0 ? j : f, kk, pr, F, g);
     }
   }
 }
@@ -774,6 +814,20 @@ struct DiagCoef {
 
 __device__ __forceinline__ double lp(const VLds& L, int s, int f, int r, int c) { return L.P[s][f][r][c]; }
 
+// the four fluxes of a face over its J (rJ = RN(1/Jf)); where one is NaN, by
+// plain divisions: div_rn's bits end where an operand is infinite or zero
+__device__ __forceinline__ void over_face_J(double o[4], double Jf, double rJ) {
+  double q[4], s = 0.0;
+#pragma unroll
+  for (int v = 0; v < 4; v++) s += q[v] = div_rn(o[v], Jf, rJ);
+  if (__builtin_expect(s != s, 0)) {
+#pragma unroll
+    for (int v = 0; v < 4; v++) q[v] = o[v] / Jf;
+  }
+#pragma unroll
+  for (int v = 0; v < 4; v++) o[v] = q[v];
+}
+
 // x face between planes (slot sm) and (slot s0) at LDS cell (r, c); the
 // face metrics of LDS row r are L.PJ[.][.][r - 1]
 __device__ __forceinline__ void vface_x(const VLds& L, int s0, int sm, int r, int c, double invXI, double inv4ET,
@@ -790,12 +844,12 @@ __device__ __forceinline__ void vface_x(const VLds& L, int s0, int sm, int r, in
   const double d5 = m.X * m.E, d7 = -((2. / 3) * m.X * m.E);
   const double e6 = m.X * m.Z, e9 = -((2. / 3) * m.X * m.Z);
   const double Ux = 0.5 * (P0.U + iP.U), Vx = 0.5 * (P0.V + iP.V), Wx = 0.5 * (P0.W + iP.W);
-  o[0] = div_rn(MU_L * (a1 * dx.u + d7 * dyv + e9 * dzw), Jf, rJ);
-  o[1] = div_rn(MU_L * (a2 * dx.v + d5 * dyu), Jf, rJ);
-  o[2] = div_rn(MU_L * (a3 * dx.w + e6 * dzu), Jf, rJ);
-  o[3] = div_rn(MU_L * (0.5 * a1 * dx.uu + 0.5 * a2 * dx.vv + 0.5 * a3 * dx.ww + CF_CVK_PR(a4, dx.T) + d5 * Vx * dyu +
-                 d7 * Ux * dyv + e6 * Wx * dzu + e9 * Ux * dzw),
-                Jf, rJ);
+  o[0] = MU_L * (a1 * dx.u + d7 * dyv + e9 * dzw);
+  o[1] = MU_L * (a2 * dx.v + d5 * dyu);
+  o[2] = MU_L * (a3 * dx.w + e6 * dzu);
+  o[3] = MU_L * (0.5 * a1 * dx.uu + 0.5 * a2 * dx.vv + 0.5 * a3 * dx.ww + CF_CVK_PR(a4, dx.T) + d5 * Vx * dyu +
+                 d7 * Ux * dyv + e6 * Wx * dzu + e9 * Ux * dzw);
+  over_face_J(o, Jf, rJ);
 }
 
 // y face between rows r-1 and r of plane slot s0
@@ -813,12 +867,12 @@ __device__ __forceinline__ void vface_y(const VLds& L, int sp, int s0, int sm, i
   const double d5 = m.X * m.E, d7 = -((2. / 3) * m.X * m.E);
   const double f8 = m.E * m.Z, f10 = -((2. / 3) * m.E * m.Z);
   const double Uy = 0.5 * (P0.U + jP.U), Vy = 0.5 * (P0.V + jP.V), Wy = 0.5 * (P0.W + jP.W);
-  o[0] = div_rn(MU_L * (d5 * dxv + b1 * dy.u), Jf, rJ);
-  o[1] = div_rn(MU_L * (d7 * dxu + b2 * dy.v + f10 * dzw), Jf, rJ);
-  o[2] = div_rn(MU_L * (b3 * dy.w + f8 * dzv), Jf, rJ);
-  o[3] = div_rn(MU_L * (0.5 * b1 * dy.uu + 0.5 * b2 * dy.vv + 0.5 * b3 * dy.ww + CF_CVK_PR(b4, dy.T) + d5 * Uy * dxv +
-                 d7 * Vy * dxu + f8 * Wy * dzv + f10 * Vy * dzw),
-                Jf, rJ);
+  o[0] = MU_L * (d5 * dxv + b1 * dy.u);
+  o[1] = MU_L * (d7 * dxu + b2 * dy.v + f10 * dzw);
+  o[2] = MU_L * (b3 * dy.w + f8 * dzv);
+  o[3] = MU_L * (0.5 * b1 * dy.uu + 0.5 * b2 * dy.vv + 0.5 * b3 * dy.ww + CF_CVK_PR(b4, dy.T) + d5 * Uy * dxv +
+                 d7 * Vy * dxu + f8 * Wy * dzv + f10 * Vy * dzw);
+  over_face_J(o, Jf, rJ);
 }
 
 // z face between columns c-1 and c of plane slot s0
@@ -836,12 +890,12 @@ __device__ __forceinline__ void vface_z(const VLds& L, int sp, int s0, int sm, i
   const double e6 = m.X * m.Z, e9 = -((2. / 3) * m.X * m.Z);
   const double f8 = m.E * m.Z, f10 = -((2. / 3) * m.E * m.Z);
   const double Uz = 0.5 * (P0.U + kP.U), Vz = 0.5 * (P0.V + kP.V), Wz = 0.5 * (P0.W + kP.W);
-  o[0] = div_rn(MU_L * (e6 * dxw + c1 * dz.u), Jf, rJ);
-  o[1] = div_rn(MU_L * (f8 * dyw + c2 * dz.v), Jf, rJ);
-  o[2] = div_rn(MU_L * (e9 * dxu + f10 * dyv + c3 * dz.w), Jf, rJ);
-  o[3] = div_rn(MU_L * (0.5 * c1 * dz.uu + 0.5 * c2 * dz.vv + 0.5 * c3 * dz.ww + CF_CVK_PR(c4, dz.T) + e6 * Uz * dxw +
-                 e9 * Wz * dxu + f8 * Vz * dyw + f10 * Wz * dyv),
-                Jf, rJ);
+  o[0] = MU_L * (e6 * dxw + c1 * dz.u);
+  o[1] = MU_L * (f8 * dyw + c2 * dz.v);
+  o[2] = MU_L * (e9 * dxu + f10 * dyv + c3 * dz.w);
+  o[3] = MU_L * (0.5 * c1 * dz.uu + 0.5 * c2 * dz.vv + 0.5 * c3 * dz.ww + CF_CVK_PR(c4, dz.T) + e6 * Uz * dxw +
+                 e9 * Wz * dxu + f8 * Vz * dyw + f10 * Wz * dyv);
+  over_face_J(o, Jf, rJ);
 }
 
 __global__ void __launch_bounds__(VTHREADS) k_visc_fused(const double* __restrict__ U,
