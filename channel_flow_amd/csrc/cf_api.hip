@@ -80,7 +80,8 @@ struct cf_ctx {
   double* Ep = nullptr;   // limiter sensors EpX, EpY, EpZ on the face layouts (3)
   double* Fw = nullptr;   // Filter workspace (FILTER_WORK_FIELDS), allocated on first use
   double* ypt = nullptr;  // Y_point j-profile (Y_m)
-  double* Sm = nullptr;   // sweep-order fields: the per-cell summary (G_N) and MR, NL, NR
+  double* Sm = nullptr;   // the sweeps' fields and hand-off slots; between sweeps its start also stages host arrays
+                          // (stage_fields) and holds the Jacobi sweeps' summary
   int* order = nullptr;   // sweep tiles in dependency order
   int* sync = nullptr;    // ticket, error flag, per-tile progress (x2 directions)
   int ntiles = 0;
@@ -135,11 +136,10 @@ struct cf_ctx {
   hipStream_t aux[3] = {nullptr, nullptr, nullptr};
   hipEvent_t fork_ev = nullptr, join_ev[3] = {nullptr, nullptr, nullptr};
   long spin_limit = 1L << 22;
-  // what the pipelined sweeps' hand-off slots hold between iterations: 1 the
-  // double sentinel, 2 the float one, 0 unknown
+  // which sweeps' hand-off slots hold the sentinel between iterations (they
+  // share memory): 1 the pipelined ones' in double, 2 in float, 3 the
+  // single-wave tiles', 0 unknown
   int hand_off = 0;
-  // the NL slots that the single-wave tiles hand across hold the sentinel
-  bool tiles_seeded = false;
   double* partial = nullptr;
   // the norms, then the two sweep error flags, in pinned memory that the last
   // reduction writes: the host's and the device's address
@@ -848,24 +848,20 @@ static int sweep_pairs(const cf_ctx* c) { return c->sweep_reuse ? std::min(c->p.
 
 // The tiled sweeps need their cross-tile slots at the sentinel and leave them
 // so: they are seeded here only when that is not known (a new context, a sweep
-// that gave up; for the single-wave tiles, whose slots are NL itself, also
-// pipelined sweeps since), eagerly and never inside a graph capture
+// that gave up, a change between the pipelined and the single-wave tiles, whose
+// slots are NL itself), eagerly and never inside a graph capture
 // (cf_inner_iteration seeds before it captures)
 static void seed_hand_off(cf_ctx* c) {
   if (c->solver != 0 || effective_schedule(c) != 0) return;
-  const int want = c->fp32 ? 2 : 1;
-  const bool tiles = c->schedule == 2;
-  if (tiles ? c->tiles_seeded : (c->hand_off == want && !c->tiles_seeded)) return;
+  const int want = c->schedule == 2 ? 3 : c->fp32 ? 2 : 1;
+  if (c->hand_off == want) return;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(c->stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return;
-  if (tiles) {
+  if (want == 3)
     cf::launch_seed_tiles(c->stream, c->Sm, c->g);
-    c->tiles_seeded = true;
-    return;
-  }
-  if (c->hand_off != want) cf::launch_seed_hand_off(c->stream, c->Sm, c->g, c->fp32);
+  else
+    cf::launch_seed_hand_off(c->stream, c->Sm, c->g, c->fp32);
   c->hand_off = want;
-  c->tiles_seeded = false;
 }
 
 static void sweeps(cf_ctx* c, double deltaT, const hipEvent_t* marks = nullptr, bool fuse_rhs = false) {
@@ -907,13 +903,11 @@ static int finish_iteration(cf_ctx* c, double er[5]) {
   int r = sync(c);
   if (r) {
     c->hand_off = 0;
-    c->tiles_seeded = false;
     return r;
   }
   for (int v = 0; v < 5; v++) er[v] = c->er_host[v];
   if (c->solver == 0 && effective_schedule(c) == 0 && (c->er_host[5] != 0. || c->er_host[6] != 0.)) {
     c->hand_off = 0;  // a sweep that gave up may leave slots without the sentinel
-    c->tiles_seeded = false;
     return fail(c, CF_ERR_TIMEOUT, "LU-SGS sweep: a tile waited past its bound for an upstream tile");
   }
   for (int v = 0; v < 5; v++)
@@ -958,7 +952,7 @@ static int dual_time_device(cf_ctx* c, double deltaT, double er[5], bool want_nl
                    want_nl ? c->NL : nullptr, g, deltaT, c->p.f_drive);
   sweeps(c, deltaT, nullptr, fuse);
   if (want_nl) {
-    if (effective_schedule(c) == 0) cf::launch_sweep_outputs(c->stream, c->Sm, c->NL, c->NR, g, c->fp32);
+    if (effective_schedule(c) == 0) cf::launch_sweep_outputs(c->stream, c->Sm, c->NL, c->NR, g, c->schedule != 2, c->fp32);
     cf::launch_copy_interior(c->stream, c->NR, c->NL, g);
   }
   update(c);

@@ -1995,7 +1995,7 @@ __device__ __forceinline__ SplitCoefT<T> coef_of(T P, T beta, T rho, T rr, T Tc,
 // (the step is clamped), so the compiler counts the loads in flight exactly
 // and waits only for the oldest.
 template <bool FWD, bool FD, class T>
-__device__ __forceinline__ void pipe_loader(PipeLds<T>& L, const T* __restrict__ S, const T* __restrict__ SRC,
+__device__ __forceinline__ void pipe_loader(PipeLds<T>& L, const T* __restrict__ S, const T* SRC,
                                             const double* __restrict__ prof, const Geo& g, const Sk& q, int tile,
                                             int TY, int r, double deltaT) {
   static_assert(PIPE_SLOTS == 4, "one loader wave per slot");
@@ -2229,7 +2229,7 @@ __device__ __forceinline__ void pipe_halo_poll(PipeLds<T>& L, T* __restrict__ H,
 // stores and loads share one counter, and a wave that waits for a load waits
 // for its earlier stores too.
 template <bool FWD, class T>
-__device__ __forceinline__ void pipe_writer(PipeLds<T>& L, T* __restrict__ DST, T* __restrict__ H, const Geo& g,
+__device__ __forceinline__ void pipe_writer(PipeLds<T>& L, T* DST, T* __restrict__ H, const Geo& g,
                                             const Sk& q, int tile, int TX, int TY) {
   const int lane = threadIdx.x & 63;
   const int a = lane & 7, b = lane >> 3;
@@ -2264,8 +2264,8 @@ __device__ __forceinline__ void pipe_writer(PipeLds<T>& L, T* __restrict__ DST, 
 }
 
 template <bool FWD, bool FD, class T>
-__device__ __forceinline__ void pipe_tile(PipeLds<T>& L, const T* __restrict__ S, const T* __restrict__ SRC,
-                                          T* __restrict__ DST, T* __restrict__ H, const T* __restrict__ E,
+__device__ __forceinline__ void pipe_tile(PipeLds<T>& L, const T* __restrict__ S, const T* SRC, T* DST,
+                                          T* __restrict__ H, const T* __restrict__ E,
                                           const double* __restrict__ prof, const Geo& g, const Sk& q, int tile,
                                           int* err, long spin_limit, double deltaT) {
   const int TX = tile % q.nTI, TY = tile / q.nTI;
@@ -2291,8 +2291,8 @@ __device__ __forceinline__ void pipe_tile(PipeLds<T>& L, const T* __restrict__ S
 }
 
 template <bool FWD, class T>
-__global__ void __launch_bounds__(PIPE_THREADS) k_sweep_pipe(const T* __restrict__ S, const T* __restrict__ SRC,
-                                                             T* __restrict__ DST, T* __restrict__ H,
+__global__ void __launch_bounds__(PIPE_THREADS) k_sweep_pipe(const T* __restrict__ S, const T* SRC, T* DST,
+                                                             T* __restrict__ H,
                                                              const T* __restrict__ E,
                                                              const double* __restrict__ prof, Geo g, Sk q,
                                                              const int* __restrict__ order, int* __restrict__ sync,
@@ -2300,7 +2300,7 @@ __global__ void __launch_bounds__(PIPE_THREADS) k_sweep_pipe(const T* __restrict
   // arrays in sweep order (Sk); S holds the DiagField summary, E its copy of
   // the x edges, H the hand-off slots
   // FWD: SRC = MR, DST = NL   (NL = D^-1 (MR - L))
-  // BWD: SRC = NL, DST = NR   (NR = NL - D^-1 U)
+  // BWD: SRC = NL, DST = NR   (NR = NL - D^-1 U); the two may be the same rows
   __shared__ PipeLds<T> L;
   if (threadIdx.x == 0) L.ticket = atomicAdd(sync, 1);
   __syncthreads();
@@ -3115,29 +3115,40 @@ long sweep_scratch_elems(const Geo& g, bool fp32) { return (G_N + 5) * sweep_lay
 
 long jacobi_summary_elems(const Geo& g) { return 6 * g.nf; }
 
-long sweep_buffer_elems(const Geo& g) {
-  const Sk q = sweep_layout(g);
-  return (G_N + 15) * q.nsk + 2 * ho_at(q, q.ntiles, 0, 0);
-}
+long sweep_buffer_elems(const Geo& g) { return (G_N + 15) * sweep_layout(g).nsk; }
 
 long sweep_update_blocks(const Geo& g) {
   Sk q = sweep_layout(g);
   return (long)((q.nsteps + 3) / 4) * q.ntiles;
 }
 
-// Sbuf holds G_N summary fields, MR, NL, NR (5 each) in sweep order, then the
-// hand-off slots and the x edges' summary, as T; a float layout uses the first half of the buffer
+// Sbuf holds G_N summary fields, MR and NL (5 each) in sweep order, then room
+// for five more: the single-wave tiles' NR or, with the pipelined sweeps, the
+// hand-off slots and the x edges' summary (two fields each).  Those put the
+// last pair's NR into MR's rows, which no one reads any more, and an earlier
+// pair's, which no one reads at all, into NL's (a row is read steps before it
+// is written).  A float layout uses the first half of the buffer.
+template <class T>
+struct SweepBuf {
+  T *S, *MR, *NL, *NR, *H, *E;
+  SweepBuf(double* Sbuf, const Sk& q, bool pipelined) {
+    S = reinterpret_cast<T*>(Sbuf);
+    MR = S + (long)G_N * q.nsk;
+    NL = MR + 5 * q.nsk;
+    H = NL + 5 * q.nsk;
+    E = H + ho_at(q, q.ntiles, 0, 0);
+    NR = pipelined ? MR : H;
+  }
+};
+static_assert(4 * HO_SLOT <= 5 * 64, "the hand-off slots and the edge copy fit in five fields");
+
 template <class T>
 static void sweeps_t(hipStream_t st, double* Ui, const double* MR, double* Sbuf, const double* prof, const Geo& g,
                      double deltaT, int n_sweeps, const int* order, int* sync, double* partial, double* er_dev,
                      double DN, long spin_limit, const hipEvent_t* marks, bool pipelined, const RhsIn* rin) {
   Sk q = sweep_layout(g);
-  T* S = reinterpret_cast<T*>(Sbuf);
-  T* MRs = S + (long)G_N * q.nsk;
-  T* NLs = MRs + 5 * q.nsk;
-  T* NRs = NLs + 5 * q.nsk;
-  T* H = NRs + 5 * q.nsk;
-  T* E = H + ho_at(q, q.ntiles, 0, 0);
+  const SweepBuf<T> b(Sbuf, q, pipelined);
+  T *S = b.S, *MRs = b.MR, *NLs = b.NL, *NRs = b.NR, *H = b.H, *E = b.E;
   if (rin)
     hipLaunchKernelGGL(k_sweep_prep_rhs<T>, dim3((q.nsteps + PR - 1) / PR, q.ntiles), dim3(PR_THREADS), 0, st, Ui, *rin,
                        prof, S, MRs, E, g, q, deltaT, sync);
@@ -3164,8 +3175,8 @@ static void sweeps_t(hipStream_t st, double* Ui, const double* MR, double* Sbuf,
                            sync + nt + 2, spin_limit, deltaT);
     }
     if (pipelined)
-      hipLaunchKernelGGL((k_sweep_pipe<false, T>), dim3(nt), dim3(PIPE_THREADS), 0, st, S, NLs, NRs, H,
-                         E, prof, g, q, order, sync + nt + 2, spin_limit, deltaT);
+      hipLaunchKernelGGL((k_sweep_pipe<false, T>), dim3(nt), dim3(PIPE_THREADS), 0, st, S, NLs,
+                         sweep + 1 < n_sweeps ? NLs : NRs, H, E, prof, g, q, order, sync + nt + 2, spin_limit, deltaT);
     if (marks) (void)hipEventRecord(marks[3 + 3 * sweep], st);
   }
   // primitive update reading NR from the sweep order
@@ -3178,8 +3189,8 @@ static void sweeps_t(hipStream_t st, double* Ui, const double* MR, double* Sbuf,
 template <class T>
 static void seed_hand_off_t(hipStream_t st, double* Sbuf, const Geo& g) {
   Sk q = sweep_layout(g);
-  T* H = reinterpret_cast<T*>(Sbuf) + (long)(G_N + 15) * q.nsk;
-  hipLaunchKernelGGL(k_seed_hand_off<T>, dim3((q.nsteps + 1) / 2, q.ntiles), dim3(256), 0, st, H, q);
+  hipLaunchKernelGGL(k_seed_hand_off<T>, dim3((q.nsteps + 1) / 2, q.ntiles), dim3(256), 0, st,
+                     SweepBuf<T>(Sbuf, q, true).H, q);
 }
 
 void launch_seed_hand_off(hipStream_t st, double* Sbuf, const Geo& g, bool fp32) {
@@ -3191,8 +3202,8 @@ void launch_seed_hand_off(hipStream_t st, double* Sbuf, const Geo& g, bool fp32)
 
 void launch_seed_tiles(hipStream_t st, double* Sbuf, const Geo& g) {
   Sk q = sweep_layout(g);
-  hipLaunchKernelGGL(k_seed_tiles, dim3((q.nsteps + 3) / 4, q.ntiles), dim3(256), 0, st, Sbuf + (long)(G_N + 5) * q.nsk,
-                     q);
+  hipLaunchKernelGGL(k_seed_tiles, dim3((q.nsteps + 3) / 4, q.ntiles), dim3(256), 0, st,
+                     SweepBuf<double>(Sbuf, q, false).NL, q);
 }
 
 void launch_sweeps(hipStream_t st, double* Ui, const double* MR, double* Sbuf, const double* prof, const Geo& g,
@@ -3207,21 +3218,20 @@ void launch_sweeps(hipStream_t st, double* Ui, const double* MR, double* Sbuf, c
 }
 
 template <class T>
-static void sweep_outputs_t(hipStream_t st, const double* Sbuf, double* NL, double* NR, const Geo& g) {
+static void sweep_outputs_t(hipStream_t st, double* Sbuf, double* NL, double* NR, const Geo& g, bool pipelined) {
   Sk q = sweep_layout(g);
-  const T* NLs = reinterpret_cast<const T*>(Sbuf) + (long)(G_N + 5) * q.nsk;
-  const T* NRs = NLs + 5 * q.nsk;
-  hipLaunchKernelGGL(k_sk_to_natural<T>, dim3((q.nsteps + 15) / 16, q.ntiles), dim3(1024), 0, st, NLs, NL, g, q, 5);
-  hipLaunchKernelGGL(k_sk_to_natural<T>, dim3((q.nsteps + 15) / 16, q.ntiles), dim3(1024), 0, st, NRs, NR, g, q, 5);
+  const SweepBuf<T> b(Sbuf, q, pipelined);
+  const dim3 gr((q.nsteps + 15) / 16, q.ntiles);
+  hipLaunchKernelGGL(k_sk_to_natural<T>, gr, dim3(1024), 0, st, b.NL, NL, g, q, 5);
+  hipLaunchKernelGGL(k_sk_to_natural<T>, gr, dim3(1024), 0, st, b.NR, NR, g, q, 5);
 }
 
-void launch_sweep_outputs(hipStream_t st, const double* Sbuf, double* NL, double* NR, const Geo& g, bool fp32) {
+void launch_sweep_outputs(hipStream_t st, double* Sbuf, double* NL, double* NR, const Geo& g, bool pipelined, bool fp32) {
   if (fp32)
-    sweep_outputs_t<float>(st, Sbuf, NL, NR, g);
+    sweep_outputs_t<float>(st, Sbuf, NL, NR, g, pipelined);
   else
-    sweep_outputs_t<double>(st, Sbuf, NL, NR, g);
+    sweep_outputs_t<double>(st, Sbuf, NL, NR, g, pipelined);
 }
-
 
 void launch_sweeps_planes(hipStream_t st, const double* Ui, const double* MR, double* NL, double* NR,
                           const double* prof, const Geo& g, double deltaT, int n_sweeps, const hipEvent_t* marks) {

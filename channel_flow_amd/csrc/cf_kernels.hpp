@@ -67,7 +67,7 @@ void launch_sweeps(hipStream_t st, double* Ui, const double* MR, double* Sbuf, c
                    double DN, long spin_limit, const hipEvent_t* marks = nullptr, bool pipelined = true,
                    const RhsIn* rin = nullptr, bool fp32 = false);
 // NL and NR of the last sweep back in the natural layout
-void launch_sweep_outputs(hipStream_t st, const double* Sbuf, double* NL, double* NR, const Geo& g, bool fp32 = false);
+void launch_sweep_outputs(hipStream_t st, double* Sbuf, double* NL, double* NR, const Geo& g, bool pipelined, bool fp32);
 // the single-wave tiles' cross-tile NL slots in Sbuf set to the sentinel
 void launch_seed_tiles(hipStream_t st, double* Sbuf, const Geo& g);
 // the pipelined sweeps' hand-off slots in Sbuf set to the sentinel
