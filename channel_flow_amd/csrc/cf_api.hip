@@ -195,8 +195,6 @@ static int stage_fields(const cf_ctx* c, long elems) {
 // order.  Small ones go through pinned memory in one copy: a copy per field
 // costs more than the bytes.
 static int stage_in(cf_ctx* c, const double* const* src, int n, long elems) {
-  for (int v = 0; v < n; v++)
-    if (!src[v]) return fail(c, CF_ERR_ARG, "null input array %d", v);
   if (n * elems <= PIN_ELEMS) {
     if (int r = sync(c)) return r;  // the pinned buffer is free
     for (int v = 0; v < n; v++) memcpy(c->pin + v * elems, src[v], elems * sizeof(double));
@@ -225,6 +223,8 @@ static int stage_out(cf_ctx* c, double* const* dst, int n, long elems) {
 
 // reference layout (Z_m pitch) <-> device layout (Zp pitch)
 static int h2d_n(cf_ctx* c, double* dst, const double* const* src, int n) {
+  for (int v = 0; v < n; v++)
+    if (!src[v]) return fail(c, CF_ERR_ARG, "null input array %d", v);
   const long elems = host_elems(c);
   const int most = stage_fields(c, elems);
   for (int v = 0; v < n; v += most) {
