@@ -852,7 +852,7 @@ static int sweep_pairs(const cf_ctx* c) { return c->sweep_reuse ? std::min(c->p.
 // slots are NL itself), eagerly and never inside a graph capture
 // (cf_inner_iteration seeds before it captures)
 static void seed_hand_off(cf_ctx* c) {
-  if (c->solver != 0 || effective_schedule(c) != 0) return;
+  if (effective_schedule(c) != 0) return;
   const int want = c->schedule == 2 ? 3 : c->fp32 ? 2 : 1;
   if (c->hand_off == want) return;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -906,7 +906,7 @@ static int finish_iteration(cf_ctx* c, double er[5]) {
     return r;
   }
   for (int v = 0; v < 5; v++) er[v] = c->er_host[v];
-  if (c->solver == 0 && effective_schedule(c) == 0 && (c->er_host[5] != 0. || c->er_host[6] != 0.)) {
+  if (c->er_host[5] != 0. || c->er_host[6] != 0.) {  // (0 where no tiled sweep ran)
     c->hand_off = 0;  // a sweep that gave up may leave slots without the sentinel
     return fail(c, CF_ERR_TIMEOUT, "LU-SGS sweep: a tile waited past its bound for an upstream tile");
   }
@@ -1160,9 +1160,10 @@ static int prepare_iteration(cf_ctx* c) {
     }
     HIPCHK(c, hipEventCreateWithFlags(&c->fork_ev, hipEventDisableTiming));
   }
-  if (c->solver == 0)
+  if (c->solver == 0) {
     if (int r = check_precision(c)) return r;
-  seed_hand_off(c);
+    seed_hand_off(c);
+  }
   return CF_OK;
 }
 
