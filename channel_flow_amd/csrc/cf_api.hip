@@ -174,7 +174,12 @@ static int fail(cf_ctx* c, int code, const char* fmt, ...) {
     if (e_ != hipSuccess) return fail((c), CF_ERR_HIP, "%s: %s", #expr, hipGetErrorString(e_)); \
   } while (0)
 
-constexpr long PIN_ELEMS = 1L << 17;  // doubles of a context's pinned buffer (1 MB)
+// doubles of a context's pinned buffer (1 MB).  Sets of fields up to that size
+// go through it in one copy, larger ones by a copy per field from the caller's
+// pages: cf_read_state of 7200 doubles 25 us against 77, of 102400 58 against
+// 92; a buffer for 2^20 would still gain above that (165760 doubles 84 us
+// against 114), for 8 MB of pinned memory a context.
+constexpr long PIN_ELEMS = 1L << 17;
 
 static long host_elems(const cf_ctx* c) { return (long)c->g.Xnp * c->g.Ym * c->g.Zm; }
 
@@ -915,7 +920,6 @@ static int finish_iteration(cf_ctx* c, double er[5]) {
   return CF_OK;
 }
 
-// the implicit part of one inner iteration on device-resident fields
 // Where the Jacobi sweeps keep their summary, or null for the general kernel:
 // it needs diagonal metrics, and room in the sweep buffer's scratch, which the
 // ghost layers of thin grids exceed (8x8x64).  Per sweep at 128x96x128: 154 us
@@ -942,6 +946,7 @@ static int dplusgs_device(cf_ctx* c, double deltaT, double er[5]) {
   return CF_OK;
 }
 
+// the implicit part of one inner iteration on device-resident fields
 static int dual_time_device(cf_ctx* c, double deltaT, double er[5], bool want_nl) {
   const Geo& g = c->g;
   if (c->solver == 1) return dplusgs_device(c, deltaT, er);
@@ -1138,9 +1143,10 @@ static bool replays_graph(const cf_ctx* c) {
 
 // Whether the stencils run on four streams.  The fork and join cost seven event
 // calls eagerly (about 30 us: 16x12x16 124 us an iteration on one stream, 155
-// on four; 64^3 337 and 357; 128x96x128 855 and 871; 256x192x256 4301 and
-// 4277) and little in a graph (48^3 256 and 263; 56^3 298 and 292; 256x192x256
-// 4311 and 4246).
+// on four; 64^3 337 and 357; 2.6 M cells 1197 and 1213; 3.7 M 1578 and 1564;
+// 4.4 M 1795 and 1802; 6.9 M 2554 and 2531; 256x192x256 4311 and 4288) and
+// little in a graph (48^3 256 and 263; 56^3 298 and 292; 256x192x256 4311 and
+// 4246).
 static bool fork_pays(const cf_ctx* c) {
   const long cells = (long)c->p.X_out * c->p.Y_out * c->p.Z_out;
   return cells >= (replays_graph(c) ? 150000 : 4000000);

@@ -815,7 +815,9 @@ struct DiagCoef {
 __device__ __forceinline__ double lp(const VLds& L, int s, int f, int r, int c) { return L.P[s][f][r][c]; }
 
 // the four fluxes of a face over its J (rJ = RN(1/Jf)); where one is NaN, by
-// plain divisions: div_rn's bits end where an operand is infinite or zero
+// plain divisions: div_rn's bits end where an operand is infinite or zero.
+// (The check takes the kernel from 467 to 481 us at 256x192x256; one check a
+// plane, with the faces formed again by a second copy of their code, 529.)
 __device__ __forceinline__ void over_face_J(double o[4], double Jf, double rJ) {
   double q[4], s = 0.0;
 #pragma unroll
@@ -2793,7 +2795,9 @@ void launch_flux_tables(hipStream_t st, double* prof, const Geo& g) {
 // time is that of one run, face after face.  Flux_X / Flux_Y: 64^3 38 / 38 us
 // with 16 faces, 16 / 16 with 1 (4160 waves); 128x96x128 62 / 60 us with 16,
 // 48 / 50 with 4 (6336); 256x192x256 438 / 434 us with 1, 322 / 329 with 16
-// (13056).
+// (13056).  The limiter fluxes, x / y, with 16 faces and with this rule: 64^3
+// 67 / 79 and 25 / 27 us, 128x96x128 118 / 135 and 96 / 107, 192x144x192
+// 333 / 379 and 311 / 350.
 static int flux_run(long rows, int nf) {
   int fc = FC;
   while (fc > 1 && rows * ((nf + fc - 1) / fc) < 6144) fc /= 2;
